@@ -56,6 +56,18 @@ __device__ __forceinline__ float max16_nn(const f32x4 (&s)[4]) {
 __device__ __forceinline__ float max8_nn(const f32x4 (&s)[2]) {
     return max_nn(max3_nn(max3_nn(s[0][0], s[0][1], s[0][2]), max3_nn(s[0][3], s[1][0], s[1][1]), s[1][2]), s[1][3]);
 }
+// max of m and 4 N accumulator values straight from the matrix cores, as
+// compiler-visible instructions (v_maximum3_f32), so that the wait states a
+// matrix result needs before a VALU reads it are placed by the compiler
+template <int N>
+__device__ __forceinline__ float max_acc(const f32x4 (&s)[N], float m) {
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, s[n][0]), s[n][1]);
+        m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, s[n][2]), s[n][3]);
+    }
+    return m;
+}
 // the maximum of a lane's scores of one block: 4 sub-tiles of 16 keys (64-key
 // block) or 2 (32-key block)
 __device__ __forceinline__ float max_sub_nn(const f32x4 (&s)[4]) { return max16_nn(s); }

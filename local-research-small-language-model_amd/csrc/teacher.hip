@@ -7,15 +7,25 @@
 // (causal: keys s <= t, blocks j > t / bs get 0), without materialising the
 // [B, Hq, T, T] weights the reference builds. bf16 inputs, D = 64, bs = 64.
 //
-// One workgroup (4 wavefronts) per (b, g, query block of 64 tokens); wavefront
+// One workgroup of NW wavefronts per (b, g, window of 16 NW tokens); wavefront
 // w owns tokens 16w .. 16w+15 for all R heads as R tiles of 16 columns (column
 // c -> token c / R, head c % R), like the sparse prefill. K blocks are staged in
 // LDS (double-buffered, the next block in flight in registers) and shared by
-// the four wavefronts; S^T = K Q^T per block and tile with
-// v_mfma_f32_16x16x32_bf16. Pass 1 walks the blocks for every column's max and
-// sum of exponentials (fp32, log2 domain); pass 2 walks them again and sums the
-// normalised probabilities of each block per column in fp32; the R columns of a
-// token are averaged through the wavefront's LDS slot and written as one value.
+// the wavefronts; S^T = K Q^T per block and tile with v_mfma_f32_16x16x32_bf16.
+// Bound by the exponentials and the matrix products of the scores, so each score
+// is formed and exponentiated once: against the column's maximum over block 0
+// (which every column attends, key 0 being allowed to every token), the block
+// sums fp32 per column in LDS, and with them the row sums; the window's rows are
+// normalised and written at the end, coalesced along the blocks. A row sum past
+// kTGuard (a score far above block 0's, whose exponent would cost precision)
+// has the workgroup take the exact column maxima and walk again. The 4
+// lane groups' partial sums of a column are added by one fp32 matrix product
+// with a selector (v_mfma_f32_16x16x4_f32, exact products with 1 and 0). Windows
+// of more than kTKeep blocks do not keep every block sum: they walk once for the
+// row sums alone and again for the block sums, written kTKeep blocks at a time.
+// B=4, T=4096, 12/4 heads: 105 us (490 TFLOP/s), from 205 us with two walks that both
+// exponentiated, a running maximum and lane-pair sums per block; B=1, T=8192
+// (two walks) 249 us, from 325.
 #include "common.h"
 #include "kernels.h"
 #include "mfma.h"
@@ -24,35 +34,38 @@ namespace sparda {
 
 constexpr int kTBs = 64;           // block size
 constexpr int kTD = 64;            // head dim
-constexpr int kTThreads = 256;
 constexpr int kTKRow = kTD + 8;    // K row in LDS (bf16 elements, 144 B)
+constexpr int kTKeep = 64;         // block sums kept per column (50 KB of LDS for 4 wavefronts, two workgroups per CU)
+constexpr int kTSRow = 49;         // LDS row of one block's column sums (odd: reads along the blocks are conflict-free)
+constexpr float kTGuard = 65536.0f; // 2^16
+constexpr int64_t kTCus = 256;
 
-template <int R>
-struct TeacherSmem {
-    uint16_t k[2][kTBs * kTKRow];
-    float colmass[4][16 * R];      // per wavefront: the block mass of each column
-};
-
-template <int R>
-__global__ void __launch_bounds__(kTThreads, 2)
+template <int R, int NW>
+__global__ void __launch_bounds__(NW * kWave, 2)
 teacher_mass_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, int64_t q_sh,
                     const uint16_t* __restrict__ k, int64_t k_sb, int64_t k_st, int64_t k_sh,
                     int64_t T, int H, int64_t NBq, int64_t NB, int causal, float scale_log2,
                     float* __restrict__ mass) {
-    __shared__ TeacherSmem<R> sm;
+    static_assert(16 * R <= kTSRow, "columns of a wavefront");
+    constexpr int kThreads = NW * kWave;
+    constexpr int kWin = 16 * NW;                // tokens per workgroup
+    constexpr int kCh = kTBs * 8 / kThreads;     // 16-byte K chunks each thread stages per block
+    __shared__ uint16_t kst[2][kTBs * kTKRow];
+    __shared__ int flag;                         // some row sum passed kTGuard
+    extern __shared__ float sums[];              // [NW][min(NB, kTKeep)][kTSRow]
     const int tid = threadIdx.x;
     const int lane = tid % kWave;
-    const int wave = tid / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int col16 = lane % 16;
     const int grp = lane / 16;
-    // heaviest query blocks first
+    // heaviest windows first
     const int64_t BH = static_cast<int64_t>(gridDim.x) / NBq;
     const int64_t bg = blockIdx.x % BH;
-    const int64_t qb = NBq - 1 - blockIdx.x / BH;
+    const int64_t t0 = (NBq - 1 - blockIdx.x / BH) * kWin;
     const int b = static_cast<int>(bg / H);
     const int g = static_cast<int>(bg % H);
-    const int64_t t0 = qb * kTBs;
-    const int64_t jmax = causal ? qb : NB - 1;
+    const int64_t t_last = t0 + kWin - 1 < T - 1 ? t0 + kWin - 1 : T - 1;
+    const int jmax = static_cast<int>(causal ? t_last / kTBs : NB - 1);
 
     // Q operands of this wavefront's tiles, straight from memory
     int tok[R];
@@ -68,110 +81,176 @@ teacher_mass_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, 
         qreg[tt][1] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(qp + 32));
     }
 
-    // K staging: chunk c = tid, tid + 256 -> row c / 8, 16-byte chunk c % 8
+    // K staging: chunk c = tid + i * kThreads -> row c / 8, 16-byte chunk c % 8;
+    // rows past T repeat row T-1 (masked)
     const uint16_t* kbase = k + b * k_sb + static_cast<int64_t>(g) * k_sh;
-    const int c_lo = tid, c_hi = tid + kTThreads;
-    const int lds_lo = (c_lo / 8) * kTKRow + (c_lo % 8) * 8, lds_hi = (c_hi / 8) * kTKRow + (c_hi % 8) * 8;
-    auto fetch = [&](int64_t j, uint4& lo, uint4& hi) {
-        int64_t s_lo = j * kTBs + c_lo / 8, s_hi = j * kTBs + c_hi / 8;
-        s_lo = s_lo < T ? s_lo : T - 1;  // rows past T repeat row T-1 (masked)
-        s_hi = s_hi < T ? s_hi : T - 1;
-        lo = *reinterpret_cast<const uint4*>(kbase + s_lo * k_st + (c_lo % 8) * 8);
-        hi = *reinterpret_cast<const uint4*>(kbase + s_hi * k_st + (c_hi % 8) * 8);
+    const int srow = tid / 8, scol = (tid % 8) * 8;
+    typedef unsigned int StageV __attribute__((ext_vector_type(4 * kCh)));
+    auto fetch = [&](int j, StageV& r) __attribute__((always_inline)) {
+        const int64_t row0 = static_cast<int64_t>(j) * kTBs;
+        const int last = static_cast<int>(T - 1 - row0 < kTBs - 1 ? T - 1 - row0 : kTBs - 1);
+        const uint16_t* kb = kbase + row0 * k_st;
+#pragma unroll
+        for (int i = 0; i < kCh; ++i) {
+            int s = srow + i * (kThreads / 8);
+            s = s < last ? s : last;
+            const uint4 a = *reinterpret_cast<const uint4*>(kb + (s * k_st + scol));
+            r[4 * i] = a.x; r[4 * i + 1] = a.y; r[4 * i + 2] = a.z; r[4 * i + 3] = a.w;
+        }
+    };
+    auto stash = [&](int buf, const StageV& r) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kCh; ++i)
+            *reinterpret_cast<uint4*>(&kst[buf][(srow + i * (kThreads / 8)) * kTKRow + scol]) =
+                uint4{r[4 * i], r[4 * i + 1], r[4 * i + 2], r[4 * i + 3]};
     };
 
-    // S^T of block j for tile tt, masked keys at -inf
-    auto scores = [&](int buf, int64_t j, int tt, f32x4 (&s)[4]) {
+    float m[R];     // the columns' references (log2 units)
+#pragma unroll
+    for (int tt = 0; tt < R; ++tt) m[tt] = -__builtin_inff();
+    float l = 0.0f;   // row sum of column col16 of tile grp (lanes with grp < R)
+    // selectors: product t adds tile t's four lane-group partials into row 4t of
+    // the result, element 0 of lane group t
+    float pick[R];
+#pragma unroll
+    for (int tt = 0; tt < R; ++tt) pick[tt] = col16 == 4 * tt ? 1.0f : 0.0f;
+
+    // S^T of block j for every tile; masked keys at -inf
+    const int64_t w_first = t0 + 16 * wave;
+    auto scores = [&](int buf, int j, f32x4 (&s)[R][4]) __attribute__((always_inline)) {
         bf16x8 ka[4][2];
 #pragma unroll
         for (int n = 0; n < 4; ++n)
 #pragma unroll
             for (int kk = 0; kk < 2; ++kk)
-                ka[n][kk] = lds_read8(&sm.k[buf][(16 * n + col16) * kTKRow + 32 * kk + 8 * grp]);
+                ka[n][kk] = lds_read8(&kst[buf][(16 * n + col16) * kTKRow + 32 * kk + 8 * grp]);
 #pragma unroll
-        for (int n = 0; n < 4; ++n) {
-            s[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-            s[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[n][0], qreg[tt][0], s[n], 0, 0, 0);
-            s[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[n][1], qreg[tt][1], s[n], 0, 0, 0);
-        }
+        for (int tt = 0; tt < R; ++tt)
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+                s[tt][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[n][0], qreg[tt][0], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                s[tt][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[n][1], qreg[tt][1], s[tt][n], 0, 0, 0);
+            }
         // causal diagonal: key <= token; any block: key < T
-        const int64_t lim_t = T - 1 - j * kTBs;
-        const int64_t lim = (causal && j == qb) ? (tok[tt] < lim_t ? tok[tt] : lim_t) : lim_t;
-        if (lim < kTBs - 1) {
+        const int64_t key0 = static_cast<int64_t>(j) * kTBs;
+        if ((causal && key0 + kTBs - 1 > w_first) || key0 + kTBs > T) {  // wave-uniform
+            const int lim_t = static_cast<int>(T - 1 - key0 < kTBs ? T - 1 - key0 : kTBs);
+            const int d0 = static_cast<int>(t0 - key0);  // causal: at least -kWin + 1
 #pragma unroll
-            for (int n = 0; n < 4; ++n)
+            for (int tt = 0; tt < R; ++tt) {
+                const int lim = causal && d0 + tok[tt] < lim_t ? d0 + tok[tt] : lim_t;
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (16 * n + 4 * grp + i > lim) s[n][i] = -__builtin_inff();
+                for (int n = 0; n < 4; ++n)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (16 * n + 4 * grp + i > lim) s[tt][n][i] = -__builtin_inff();
+            }
         }
     };
 
-    float m[R], l[R];
+    const int keep = static_cast<int>(NB < kTKeep ? NB : kTKeep);
+    const bool once = jmax < kTKeep;  // every block sum is kept: one walk
+    float* ws = sums + static_cast<int64_t>(wave) * keep * kTSRow;
+    // normalises and writes blocks [j0, j1) of the wavefront's rows from `ws`
+    // (filled by this wavefront alone): lane -> block j0 + lane
+    auto flush = [&](int j0, int j1) __attribute__((always_inline)) {
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll 2
+        for (int tk = 0; tk < 16; ++tk) {
+            const int64_t t = w_first + tk;
+            if (t >= T) break;  // wave-uniform
+            float v = 0.0f;
+            const int row = j0 + lane < j1 ? lane : 0;
 #pragma unroll
-    for (int tt = 0; tt < R; ++tt) {
-        m[tt] = -__builtin_inff();
-        l[tt] = 0.0f;
-    }
+            for (int hh = 0; hh < R; ++hh) {
+                const int c = R * tk + hh;
+                // the column's row sum sits in lane c (tile c / 16, column c % 16)
+                const float lc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, l), c));
+                v += ws[row * kTSRow + c] / lc;
+            }
+            if (j0 + lane < j1)
+                mass[((static_cast<int64_t>(b) * H + g) * T + t) * NB + j0 + lane] = v / static_cast<float>(R);
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
 
-    for (int pass = 0; pass < 2; ++pass) {
-        uint4 ka_lo, ka_hi;
-        fetch(0, ka_lo, ka_hi);
-        __syncthreads();  // the previous pass has read its last buffer
-        *reinterpret_cast<uint4*>(&sm.k[0][lds_lo]) = ka_lo;
-        *reinterpret_cast<uint4*>(&sm.k[0][lds_hi]) = ka_hi;
-        if (jmax >= 1) fetch(1, ka_lo, ka_hi);
+    // one pass over the blocks. maxima: the exact column maxima (lane-local) into
+    // m; else the block sums against m (set from block 0 unless `exact`): added
+    // into l (count) and kept, written when kTKeep of them are held (store)
+    auto walk = [&](bool maxima, bool exact, bool count, bool store) __attribute__((always_inline)) {
+        StageV nk{};
+        fetch(0, nk);
+        __syncthreads();  // the previous walk has read its last buffer
+        stash(0, nk);
+        if (jmax >= 1) fetch(1, nk);
         __syncthreads();
-        for (int64_t j = 0; j <= jmax; ++j) {
-            const int buf = static_cast<int>(j & 1);
+        int j0 = 0;  // first block held in `ws`
+        for (int j = 0; j <= jmax; ++j) {
+            const int buf = j & 1;
+            f32x4 s[R][4];
+            scores(buf, j, s);
+            if (maxima) {
 #pragma unroll
-            for (int tt = 0; tt < R; ++tt) {
-                f32x4 s[4];
-                scores(buf, j, tt, s);
-                if (pass == 0) {
-                    float mx = pair32_max(pair16_max(max16_nn(s))) * scale_log2;
-                    const float m_new = __builtin_fmaxf(m[tt], mx);
-                    float acc = 0.0f;
+                for (int tt = 0; tt < R; ++tt) m[tt] = max_acc(s[tt], m[tt]);
+            } else {
+                if (j == 0 && !exact) {  // wave-uniform
 #pragma unroll
-                    for (int n = 0; n < 4; ++n)
+                    for (int tt = 0; tt < R; ++tt)
+                        m[tt] = pair32_max(pair16_max(max_acc(s[tt], -__builtin_inff()))) * scale_log2;
+                }
+                f32x4 d{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            acc += __builtin_amdgcn_exp2f(__builtin_fmaf(s[n][i], scale_log2, -m_new));
-                    acc = pair32_sum(pair16_sum(acc));
-                    l[tt] = l[tt] * (m_new == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(m[tt] - m_new)) + acc;
-                    m[tt] = m_new;
-                } else {
-                    float acc = 0.0f;
+                for (int tt = 0; tt < R; ++tt) {
+                    float a[4];
 #pragma unroll
-                    for (int n = 0; n < 4; ++n)
+                    for (int n = 0; n < 4; ++n) {
+                        a[n] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[tt][n][0], scale_log2, -m[tt]));
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            acc += __builtin_amdgcn_exp2f(__builtin_fmaf(s[n][i], scale_log2, -m[tt]));
-                    acc = pair32_sum(pair16_sum(acc));
-                    if (grp == 0) sm.colmass[wave][16 * tt + col16] = acc / l[tt];
+                        for (int i = 1; i < 4; ++i)
+                            a[n] += __builtin_amdgcn_exp2f(__builtin_fmaf(s[tt][n][i], scale_log2, -m[tt]));
+                    }
+                    d = __builtin_amdgcn_mfma_f32_16x16x4f32(pick[tt], (a[0] + a[1]) + (a[2] + a[3]), d, 0, 0, 0);
+                }
+                if (count) l += d[0];
+                if (store) {
+                    if (lane < 16 * R) ws[(j - j0) * kTSRow + lane] = d[0];
+                    if (!once && j - j0 == kTKeep - 1) {  // wave-uniform
+                        flush(j0, j + 1);
+                        j0 = j + 1;
+                    }
                 }
             }
-            if (pass == 1 && lane < 16) {
-                // average of the R head columns of token 16*wave + lane
-                float v = 0.0f;
-#pragma unroll
-                for (int hh = 0; hh < R; ++hh) v += sm.colmass[wave][R * lane + hh];
-                const int64_t t = t0 + 16 * wave + lane;
-                if (t < T) mass[((static_cast<int64_t>(b) * H + g) * T + t) * NB + j] = v / static_cast<float>(R);
-            }
             if (j + 1 <= jmax) {
-                *reinterpret_cast<uint4*>(&sm.k[buf ^ 1][lds_lo]) = ka_lo;
-                *reinterpret_cast<uint4*>(&sm.k[buf ^ 1][lds_hi]) = ka_hi;
-                if (j + 2 <= jmax) fetch(j + 2, ka_lo, ka_hi);
+                stash(buf ^ 1, nk);
+                if (j + 2 <= jmax) fetch(j + 2, nk);
             }
             __syncthreads();
         }
+        if (store && !once) flush(j0, jmax + 1);
+    };
+    if (tid == 0) flag = 0;  // ordered before its uses by the walk's barriers
+    walk(false, false, true, once);
+    const bool bad = lane < 16 * R && !(l <= kTGuard);
+    if (__ballot(bad) != 0ull && lane == 0) atomicOr(&flag, 1);
+    __syncthreads();
+    if (flag != 0) {  // workgroup-uniform
+#pragma unroll
+        for (int tt = 0; tt < R; ++tt) m[tt] = -__builtin_inff();
+        walk(true, true, false, false);
+#pragma unroll
+        for (int tt = 0; tt < R; ++tt) m[tt] = pair32_max(pair16_max(m[tt])) * scale_log2;
+        l = 0.0f;
+        walk(false, true, true, once);
     }
+    if (once) flush(0, jmax + 1);
+    else walk(false, true, false, true);
     // blocks past the causal limit carry no probability
-    if (jmax + 1 < NB && lane < 16) {
-        const int64_t t = t0 + 16 * wave + lane;
-        if (t < T) {
+    if (jmax + 1 < NB) {
+        for (int tk = 0; tk < 16; ++tk) {
+            const int64_t t = w_first + tk;
+            if (t >= T) break;
             float* row = mass + ((static_cast<int64_t>(b) * H + g) * T + t) * NB;
-            for (int64_t j = jmax + 1; j < NB; ++j) row[j] = 0.0f;
+            for (int64_t j = jmax + 1 + lane; j < NB; j += kWave) row[j] = 0.0f;
         }
     }
 }
@@ -179,21 +258,30 @@ teacher_mass_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, 
 int launch_teacher_mass(const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sb,
                         int64_t k_st, int64_t k_sh, int64_t B, int64_t T, int64_t Hq, int64_t Hkv, int causal,
                         float scale, float* mass, hipStream_t stream) {
-    const int64_t NBq = cdiv(T, kTBs);
-    const int64_t NB = NBq;
+    const int64_t NB = cdiv(T, kTBs);
     const float scale_log2 = scale * 1.4426950408889634f;
-    dim3 grid(static_cast<unsigned>(B * Hkv * NBq));
     const int R = static_cast<int>(Hq / Hkv);
-#define SPARDA_TEACHER(R_)                                                                                  \
-    hipLaunchKernelGGL((teacher_mass_kernel<R_>), grid, dim3(kTThreads), 0, stream,                         \
+    // windows of 64 tokens (K staged once for four wavefronts), of 32 where those
+    // would leave the chip with fewer than two workgroups per CU, which is what
+    // the LDS of a full window allows
+    const int nw = B * Hkv * cdiv(T, 64) >= 2 * kTCus ? 4 : 2;
+    const int64_t NBq = cdiv(T, 16 * nw);
+    const size_t lds = static_cast<size_t>(nw) * (NB < kTKeep ? NB : kTKeep) * kTSRow * sizeof(float);
+    dim3 grid(static_cast<unsigned>(B * Hkv * NBq));
+#define SPARDA_TEACHER(R_, NW_)                                                                             \
+    hipLaunchKernelGGL((teacher_mass_kernel<R_, NW_>), grid, dim3(NW_ * kWave), lds, stream,                \
                        static_cast<const uint16_t*>(q), q_sb, q_st, q_sh, static_cast<const uint16_t*>(k),  \
                        k_sb, k_st, k_sh, T, static_cast<int>(Hkv), NBq, NB, causal, scale_log2, mass)
+#define SPARDA_TEACHER_W(R_)          \
+    if (nw == 4) SPARDA_TEACHER(R_, 4); \
+    else SPARDA_TEACHER(R_, 2);
     switch (R) {
-        case 1: SPARDA_TEACHER(1); break;
-        case 2: SPARDA_TEACHER(2); break;
-        case 3: SPARDA_TEACHER(3); break;
+        case 1: SPARDA_TEACHER_W(1); break;
+        case 2: SPARDA_TEACHER_W(2); break;
+        case 3: SPARDA_TEACHER_W(3); break;
         default: return set_error(SPARDA_ERR_SHAPE, "teacher_mass: Hq/Hkv = %d not in {1, 2, 3}", R);
     }
+#undef SPARDA_TEACHER_W
 #undef SPARDA_TEACHER
     return check_hip(hipGetLastError(), "teacher_mass_kernel");
 }

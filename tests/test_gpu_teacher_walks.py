@@ -1,0 +1,34 @@
+"""The teacher block mass over its workgroup shapes and walks: window edges,
+more blocks than a window keeps (row sums first, block sums in parts), and
+a score far above block 0's (the exact maxima and a second walk). fp32 sums of
+at most T terms: 1e-6 per probability against float64."""
+
+import numpy as np
+import pytest
+import torch
+
+import sparda
+from oracle import sparda_oracle as O
+from helpers import np32
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("B,T,Hq,Hkv,causal,hot", [
+    (1, 31, 12, 4, True, False), (1, 33, 8, 4, False, False), (1, 64, 4, 4, True, False),
+    (33, 250, 12, 4, True, False),            # 64-token windows, ragged
+    (1, 4161, 3, 1, True, False), (1, 4161, 1, 1, False, False),  # 66 blocks: written in parts
+    (1, 300, 12, 4, True, True), (1, 4161, 3, 1, True, True)])
+def test_teacher_mass_shapes(B, T, Hq, Hkv, causal, hot):
+    print(f"[case] teacher walks B={B} T={T} Hq={Hq} Hkv={Hkv} causal={causal} hot={hot}", flush=True)
+    g = torch.Generator().manual_seed(T + Hq)
+    q = torch.randn(B, T, Hq, 64, generator=g)
+    k = torch.randn(B, T, Hkv, 64, generator=g)
+    if hot:
+        q[0, T - 20], k[0, T - 90] = 1.5, 3.0  # 288 / 8 = 52 log2-units above a zero score
+    q, k = q.to(torch.bfloat16), k.to(torch.bfloat16)
+    got = sparda.teacher_block_mass(q.to(DEV), k.to(DEV), 64, causal=causal).cpu().numpy()
+    want = O.teacher_block_mass(np32(q[-1:]), np32(k[-1:]), 64, causal)
+    assert np.abs(got[-1:] - want).max() < 1e-6 * (4 if hot else 1)
+    assert np.abs(got.sum(-1) - 1.0).max() < 1e-5
