@@ -12,30 +12,36 @@
 // epilogue (pairs (i, i + D/2) of a head, fp32 cos / sin tables), and every
 // region is written in its own [M, heads * D] layout.
 //
-// Tiling (D = 64): a 256-thread workgroup computes a 128 x 128 tile of y, each
-// wavefront 64 x 64 = one head of one region, as 4 x 4 tiles of
-// v_mfma_f32_16x16x32_bf16. A and B (rows of x and of W', both row-major over
-// c) are staged per 32-wide step of c in LDS, the next step in flight in
-// registers. In the MFMA result layout lane l holds column l % 16 of a tile, so
-// the rotation partner of column i (i + 32 or i - 32) is in the same lane, two
-// tiles away.
+// Tiling (D = 64): a 256-thread workgroup computes a BM x 128 tile of y
+// (BM = 32 TM), each wavefront 16 TM x 64 = one head of one region, as the
+// transposed product W' x^T in 4 x TM tiles of v_mfma_f32_16x16x32_bf16 (rows
+// of W' are the A operand, rows of x the B operand). Both are staged per
+// BK-wide step of c in LDS, the next step in flight in registers. W' rows are
+// staged permuted (w_row), so that the tile pair (2p, 2p + 1) gives lane
+// l the eight consecutive columns 32p + 8 (l / 16) + 0..7 of row l % 16: the
+// outputs are 16-byte stores, and the rotation partner of a column (i + 32 or
+// i - 32) sits in the same lane, one pair away. sum(x^2) is the diagonal of
+// x x^T, formed on the matrix cores from the staged x fragments (each of the
+// two wavefronts that share the rows takes every second row tile).
+// Bound by the latency of a step's loads and LDS reads (the matrix cores are busy
+// a third of the time): 62 us = 630 TFLOP/s at M = 16384, N = 1536, C = 768, from
+// 72 us with 128 x 128 tiles, the squares on the VALU and 2-byte stores.
 #include "common.h"
 #include "kernels.h"
-#include "mfma.h"
 #include "rows.h"
 
 namespace sparda {
 
-constexpr int kPBM = 128;          // rows of y per workgroup
 constexpr int kPBN = 128;          // columns of y per workgroup
-constexpr int kPBK = 32;           // reduction step
-constexpr int kPRow = kPBK + 8;    // LDS row (bf16 elements): 80 B, 16-B aligned
 constexpr int kPThreads = 256;
+constexpr int64_t kPCus = 256;
 
+template <int TM, int BK>
 struct ProduceSmem {
-    uint16_t a[2][kPBM * kPRow];
-    uint16_t b[2][kPBN * kPRow];
-    float inv_rms[kPBM];
+    static constexpr int kRow = BK + 8;          // LDS row (bf16 elements): 80 or 144 B, 16-B aligned
+    uint16_t a[2][32 * TM * kRow];               // x rows
+    uint16_t b[2][kPBN * kRow];                  // W' rows, permuted
+    float inv_rms[32 * TM];
 };
 
 template <int ODT>
@@ -47,87 +53,155 @@ __device__ __forceinline__ void store_out(void* out, int64_t i, float v) {
     }
 }
 
-template <int FDT>
+// eight consecutive outputs; vec: the address is 16-byte aligned
+template <int ODT>
+__device__ __forceinline__ void store_out8(void* out, int64_t i, const float (&y)[8], bool vec) {
+    if (vec) {
+        if constexpr (ODT == SPARDA_F32) {
+            float4* p = reinterpret_cast<float4*>(static_cast<float*>(out) + i);
+            p[0] = make_float4(y[0], y[1], y[2], y[3]);
+            p[1] = make_float4(y[4], y[5], y[6], y[7]);
+        } else {
+            bf16x8 w;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) w[e] = static_cast<__bf16>(y[e]);
+            *reinterpret_cast<bf16x8*>(static_cast<__bf16*>(out) + i) = w;
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) store_out<ODT>(out, i + e, y[e]);
+    }
+}
+
+// eight consecutive table entries; vec: the address is 16-byte aligned
+__device__ __forceinline__ void load_tab8(const float* __restrict__ p, float (&o)[8], bool vec) {
+    if (vec) {
+        const float4 u = reinterpret_cast<const float4*>(p)[0], w = reinterpret_cast<const float4*>(p)[1];
+        o[0] = u.x; o[1] = u.y; o[2] = u.z; o[3] = u.w;
+        o[4] = w.x; o[5] = w.y; o[6] = w.z; o[7] = w.w;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = p[e];
+    }
+}
+
+// LDS row r of a 64-column head holds W' row w_row(r) of the head: tile t = r / 16,
+// row 4 g + i of it -> column 32 (t / 2) + 8 g + 4 (t % 2) + i
+__device__ __forceinline__ int w_row(int r) {
+    return (r & ~63) + 32 * ((r >> 5) & 1) + 8 * ((r >> 2) & 3) + 4 * ((r >> 4) & 1) + (r & 3);
+}
+
+template <int FDT, int TM, int BK>
 __global__ void __launch_bounds__(kPThreads, 2)
 produce_kernel(const uint16_t* __restrict__ x, int64_t x_st, const uint16_t* __restrict__ w,
                int64_t M, int C, int Nq, int Nk, int Nf, float eps,
                const float* __restrict__ cosv, const float* __restrict__ sinv, int64_t T, int64_t pos0,
                uint16_t* __restrict__ q, uint16_t* __restrict__ k, uint16_t* __restrict__ v,
-               void* __restrict__ f, const int64_t* __restrict__ pos_dev, int64_t rope_len) {
-    __shared__ ProduceSmem sm;
+               void* __restrict__ f, const int64_t* __restrict__ pos_dev, int64_t rope_len, int vec_out,
+               int vec_tab) {
+    using Smem = ProduceSmem<TM, BK>;
+    constexpr int kBM = 32 * TM;
+    constexpr int kRow = Smem::kRow;
+    constexpr int kCpr = BK / 8;                      // 16-byte chunks per row
+    constexpr int kRps = kPThreads / kCpr;            // rows staged per round
+    constexpr int kA = kBM / kRps, kB = kPBN / kRps;  // rounds
+    __shared__ Smem sm;
     const int tid = threadIdx.x;
     const int lane = tid % kWave;
-    const int wave = tid / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int col16 = lane % 16;
     const int grp = lane / 16;
-    const int wm = wave / 2, wn = wave % 2;          // 2 x 2 wavefronts of 64 x 64
-    const int64_t m0 = static_cast<int64_t>(blockIdx.x) * kPBM;
+    const int wm = wave / 2, wn = wave % 2;          // 2 x 2 wavefronts of 16 TM x 64
+    const int64_t m0 = static_cast<int64_t>(blockIdx.x) * kBM;
     const int n0 = blockIdx.y * kPBN;
 
-    // staging: 128 rows x 32 c = 512 chunks of 16 B per operand, two per thread
-    const int r_lo = tid / 4, r_hi = tid / 4 + 64, cc = (tid % 4) * 8;
-    int64_t ra_lo = m0 + r_lo, ra_hi = m0 + r_hi;
-    ra_lo = ra_lo < M ? ra_lo : M - 1;                // rows past M repeat row M-1 (not stored)
-    ra_hi = ra_hi < M ? ra_hi : M - 1;
-    const uint16_t* xa_lo = x + ra_lo * x_st + cc;
-    const uint16_t* xa_hi = x + ra_hi * x_st + cc;
-    const uint16_t* wb_lo = w + static_cast<int64_t>(n0 + r_lo) * C + cc;
-    const uint16_t* wb_hi = w + static_cast<int64_t>(n0 + r_hi) * C + cc;
-    uint4 a_lo = *reinterpret_cast<const uint4*>(xa_lo);
-    uint4 a_hi = *reinterpret_cast<const uint4*>(xa_hi);
-    uint4 b_lo = *reinterpret_cast<const uint4*>(wb_lo);
-    uint4 b_hi = *reinterpret_cast<const uint4*>(wb_hi);
+    // staging: thread -> 16-byte chunk tid % kCpr of rows tid / kCpr + i kRps
+    const int sr = tid / kCpr, cc = (tid % kCpr) * 8;
+    const int m_last = static_cast<int>(M - 1 - m0 < kBM - 1 ? M - 1 - m0 : kBM - 1);
+    const uint16_t* xa[kA];
+    const uint16_t* wb[kB];
+#pragma unroll
+    for (int i = 0; i < kA; ++i) {
+        const int r = sr + i * kRps;
+        xa[i] = x + (m0 + (r < m_last ? r : m_last)) * x_st + cc;  // rows past M repeat row M-1 (not stored)
+    }
+#pragma unroll
+    for (int i = 0; i < kB; ++i) wb[i] = w + static_cast<int64_t>(n0 + w_row(sr + i * kRps)) * C + cc;
+    typedef unsigned int StageA __attribute__((ext_vector_type(4 * kA)));
+    typedef unsigned int StageB __attribute__((ext_vector_type(4 * kB)));
+    StageA ra;
+    StageB rb;
+    auto fetch = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kA; ++i) {
+            const uint4 t = *reinterpret_cast<const uint4*>(xa[i] + c);
+            ra[4 * i] = t.x; ra[4 * i + 1] = t.y; ra[4 * i + 2] = t.z; ra[4 * i + 3] = t.w;
+        }
+#pragma unroll
+        for (int i = 0; i < kB; ++i) {
+            const uint4 t = *reinterpret_cast<const uint4*>(wb[i] + c);
+            rb[4 * i] = t.x; rb[4 * i + 1] = t.y; rb[4 * i + 2] = t.z; rb[4 * i + 3] = t.w;
+        }
+    };
+    fetch(0);
 
-    f32x4 acc[4][4];
+    f32x4 acc[4][TM];  // [W' tile][x tile]: column 16 tn + 4 grp + i (permuted), row 16 tm + col16
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float ss[4] = {0.f, 0.f, 0.f, 0.f};  // sum of squares of row 16*tm + col16 (this lane's k slice)
+        for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 sq[TM / 2];  // x x^T of the row tiles 2 t + wn
+#pragma unroll
+    for (int j = 0; j < TM / 2; ++j) sq[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int steps = C / kPBK;
+    const int steps = C / BK;
     for (int st = 0; st < steps; ++st) {
         const int buf = st & 1;
-        *reinterpret_cast<uint4*>(&sm.a[buf][r_lo * kPRow + cc]) = a_lo;
-        *reinterpret_cast<uint4*>(&sm.a[buf][r_hi * kPRow + cc]) = a_hi;
-        *reinterpret_cast<uint4*>(&sm.b[buf][r_lo * kPRow + cc]) = b_lo;
-        *reinterpret_cast<uint4*>(&sm.b[buf][r_hi * kPRow + cc]) = b_hi;
+#pragma unroll
+        for (int i = 0; i < kA; ++i)
+            *reinterpret_cast<uint4*>(&sm.a[buf][(sr + i * kRps) * kRow + cc]) =
+                uint4{ra[4 * i], ra[4 * i + 1], ra[4 * i + 2], ra[4 * i + 3]};
+#pragma unroll
+        for (int i = 0; i < kB; ++i)
+            *reinterpret_cast<uint4*>(&sm.b[buf][(sr + i * kRps) * kRow + cc]) =
+                uint4{rb[4 * i], rb[4 * i + 1], rb[4 * i + 2], rb[4 * i + 3]};
         __syncthreads();
-        if (st + 1 < steps) {
-            const int c1 = (st + 1) * kPBK;
-            a_lo = *reinterpret_cast<const uint4*>(xa_lo + c1);
-            a_hi = *reinterpret_cast<const uint4*>(xa_hi + c1);
-            b_lo = *reinterpret_cast<const uint4*>(wb_lo + c1);
-            b_hi = *reinterpret_cast<const uint4*>(wb_hi + c1);
-        }
-        bf16x8 af[4], bfr[4];
+        if (st + 1 < steps) fetch((st + 1) * BK);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            af[t] = lds_read8(&sm.a[buf][(64 * wm + 16 * t + col16) * kPRow + 8 * grp]);
-            bfr[t] = lds_read8(&sm.b[buf][(64 * wn + 16 * t + col16) * kPRow + 8 * grp]);
-        }
+        for (int kk = 0; kk < BK / 32; ++kk) {
+            bf16x8 af[TM], bfr[4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+            for (int t = 0; t < 4; ++t)
+                bfr[t] = lds_read8(&sm.b[buf][(64 * wn + 16 * t + col16) * kRow + 32 * kk + 8 * grp]);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float xv = static_cast<float>(af[t][e]);
-                ss[t] = __builtin_fmaf(xv, xv, ss[t]);
+            for (int t = 0; t < TM; ++t)
+                af[t] = lds_read8(&sm.a[buf][(16 * TM * wm + 16 * t + col16) * kRow + 32 * kk + 8 * grp]);
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                for (int tn = 0; tn < 4; ++tn)
+                    acc[tn][tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[tn], af[tm], acc[tn][tm], 0, 0, 0);
+            if (wn == 0) {  // wave-uniform
+#pragma unroll
+                for (int t = 0; t < TM / 2; ++t)
+                    sq[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[2 * t], af[2 * t], sq[t], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int t = 0; t < TM / 2; ++t)
+                    sq[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[2 * t + 1], af[2 * t + 1], sq[t], 0, 0, 0);
             }
         }
-#pragma unroll
-        for (int tm = 0; tm < 4; ++tm)
-#pragma unroll
-            for (int tn = 0; tn < 4; ++tn)
-                acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[tm], bfr[tn], acc[tm][tn], 0, 0, 0);
         // the buffer written next step was last read before this step's barrier
     }
 
-    // 1/rms of the workgroup's rows: the 4 lane groups hold disjoint c slices
-    if (wn == 0) {
+    // 1/rms of the workgroup's rows: row r of a tile is element r % 4 of lane r + 16 (r / 4)
+    if (col16 / 4 == grp) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            float s = pair32_sum(pair16_sum(ss[t]));
-            if (grp == 0) sm.inv_rms[64 * wm + 16 * t + col16] = 1.0f / __builtin_sqrtf(s / static_cast<float>(C) + eps);
+        for (int t = 0; t < TM / 2; ++t) {
+            float s = sq[t][0];
+#pragma unroll
+            for (int e = 1; e < 4; ++e) s = col16 % 4 == e ? sq[t][e] : s;
+            sm.inv_rms[16 * TM * wm + 16 * (2 * t + wn) + col16] = 1.0f / __builtin_sqrtf(s / static_cast<float>(C) + eps);
         }
     }
     __syncthreads();
@@ -146,39 +220,38 @@ produce_kernel(const uint16_t* __restrict__ x, int64_t x_st, const uint16_t* __r
     const int64_t pos_base = pos0 + (pos_dev != nullptr ? *pos_dev : 0);
     const int64_t pos_hi = pos_dev != nullptr ? rope_len - 1 : INT64_MAX;
 #pragma unroll
-    for (int tm = 0; tm < 4; ++tm) {
+    for (int tm = 0; tm < TM; ++tm) {
+        const int rloc = 16 * (TM * wm + tm) + col16;
+        const int64_t m = m0 + rloc;
+        if (m >= M) continue;
+        const float sc = sm.inv_rms[rloc];
+        float y[2][8];                               // columns 32 p + 8 grp + 0..7
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int rloc = 64 * wm + 16 * tm + 4 * grp + i;
-            const int64_t m = m0 + rloc;
-            if (m >= M) continue;
-            const float sc = sm.inv_rms[rloc];
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) y[p][e] = acc[2 * p + e / 4][tm][e % 4] * sc;
+        if (region <= 1) {
             int64_t t = t_first + rloc;
             while (t >= T) t -= T;
             int64_t pos = pos_base + t;
             pos = pos < 0 ? 0 : (pos > pos_hi ? pos_hi : pos);
-            float y[4];
+            float cs[8], sn[8];
+            load_tab8(cosv + pos * 32 + 8 * grp, cs, vec_tab != 0);
+            load_tab8(sinv + pos * 32 + 8 * grp, sn, vec_tab != 0);
 #pragma unroll
-            for (int tn = 0; tn < 4; ++tn) y[tn] = acc[tm][tn][i] * sc;
-            if (region <= 1) {
-                // columns d = 16*tn + col16: pairs (d, d + 32) are tiles (0, 2) and (1, 3)
-#pragma unroll
-                for (int tn = 0; tn < 2; ++tn) {
-                    const int d = 16 * tn + col16;
-                    const float c = cosv[pos * 32 + d], s = sinv[pos * 32 + d];
-                    const float x1 = y[tn], x2 = y[tn + 2];
-                    y[tn] = x1 * c - x2 * s;
-                    y[tn + 2] = x2 * c + x1 * s;
-                }
+            for (int e = 0; e < 8; ++e) {
+                const float x1 = y[0][e], x2 = y[1][e];
+                y[0][e] = x1 * cs[e] - x2 * sn[e];
+                y[1][e] = x2 * cs[e] + x1 * sn[e];
             }
-            const int64_t base = m * ld + 64 * head + col16;
+        }
 #pragma unroll
-            for (int tn = 0; tn < 4; ++tn) {
-                if (region == 0) store_out<SPARDA_BF16>(q, base + 16 * tn, y[tn]);
-                else if (region == 1) store_out<SPARDA_BF16>(k, base + 16 * tn, y[tn]);
-                else if (region == 2) store_out<SPARDA_BF16>(v, base + 16 * tn, y[tn]);
-                else store_out<FDT>(f, base + 16 * tn, y[tn]);
-            }
+        for (int p = 0; p < 2; ++p) {
+            const int64_t base = m * ld + 64 * head + 32 * p + 8 * grp;
+            if (region == 0) store_out8<SPARDA_BF16>(q, base, y[p], vec_out != 0);
+            else if (region == 1) store_out8<SPARDA_BF16>(k, base, y[p], vec_out != 0);
+            else if (region == 2) store_out8<SPARDA_BF16>(v, base, y[p], vec_out != 0);
+            else store_out8<FDT>(f, base, y[p], vec_out != 0);
         }
     }
 }
@@ -282,15 +355,37 @@ int launch_produce(const void* x, int64_t x_st, const void* w, int64_t M, int64_
     }
     if (kc != nullptr) return set_error(SPARDA_ERR_SHAPE, "produce: cache rows are written for M <= %d only",
                                         kRowsMaxM);
-    dim3 grid(static_cast<unsigned>(cdiv(M, kPBM)), static_cast<unsigned>(N / kPBN));
-#define SPARDA_PRODUCE(FDT_)                                                                              \
-    hipLaunchKernelGGL((produce_kernel<FDT_>), grid, dim3(kPThreads), 0, stream,                          \
+    auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+    const int vec_out = al16(q) && al16(k) && al16(v) && al16(f);  // rows are multiples of 64 elements
+    const int vec_tab = al16(cosv) && al16(sinv);
+#define SPARDA_PRODUCE(FDT_, TM_, BK_)                                                                     \
+    hipLaunchKernelGGL((produce_kernel<FDT_, TM_, BK_>),                                                   \
+                       dim3(static_cast<unsigned>(cdiv(M, 32 * TM_)), static_cast<unsigned>(N / kPBN)),    \
+                       dim3(kPThreads), 0, stream,                                                         \
                        static_cast<const uint16_t*>(x), x_st, static_cast<const uint16_t*>(w), M,        \
                        static_cast<int>(C), static_cast<int>(Nq), static_cast<int>(Nk),                   \
                        static_cast<int>(Nf), eps, cosv, sinv, T, pos0, static_cast<uint16_t*>(q),         \
-                       static_cast<uint16_t*>(k), static_cast<uint16_t*>(v), f, pos_dev, rope_len)
-    if (f_dtype == SPARDA_F32) SPARDA_PRODUCE(SPARDA_F32);
-    else SPARDA_PRODUCE(SPARDA_BF16);
+                       static_cast<uint16_t*>(k), static_cast<uint16_t*>(v), f, pos_dev, rope_len,        \
+                       vec_out, vec_tab)
+#define SPARDA_PRODUCE_T(FDT_)                                  \
+    switch (tile) {                                             \
+        case 0: SPARDA_PRODUCE(FDT_, 8, 32); break;             \
+        case 1: SPARDA_PRODUCE(FDT_, 4, 64); break;             \
+        case 2: SPARDA_PRODUCE(FDT_, 2, 64); break;             \
+        case 3: SPARDA_PRODUCE(FDT_, 4, 32); break;             \
+        default: SPARDA_PRODUCE(FDT_, 2, 32); break;            \
+    }
+    // The widest tile that leaves the chip enough workgroups (N = 1536, C = 768):
+    // 256 rows past two workgroups per CU (62 us against 74 with 128 rows at
+    // M = 16384; 39.9 against 38.7 at 8192), 128 rows past one per CU (25.9 us
+    // against 28.1 with 64 rows at 4096), 64 rows below (20.1 against 19.3 at 2048,
+    // launch included). A width that is no multiple of 64 takes 32-wide steps.
+    const int64_t cols = N / kPBN;
+    const int tile = C % 64 != 0 ? (cdiv(M, 128) * cols > kPCus ? 3 : 4)
+                                 : (cdiv(M, 256) * cols > 2 * kPCus ? 0 : (cdiv(M, 128) * cols > kPCus ? 1 : 2));
+    if (f_dtype == SPARDA_F32) { SPARDA_PRODUCE_T(SPARDA_F32) }
+    else { SPARDA_PRODUCE_T(SPARDA_BF16) }
+#undef SPARDA_PRODUCE_T
 #undef SPARDA_PRODUCE
     return check_hip(hipGetLastError(), "produce_kernel");
 }
