@@ -224,6 +224,16 @@ int offload_append_at(sparda_offload_t h, const void* k, const void* v, int64_t 
                       const int64_t* pos_dev, int64_t bs, float* sums, hipStream_t stream,
                       const PrefetchDev* pf = nullptr);
 
+// fp32 on the matrix cores (D = 64, blocks of 64 or 32 keys); sel nullptr: dense
+bool prefill_f32_supported(int dtype, int64_t T, int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int64_t B,
+                           const int32_t* sel, int64_t q_sb, int64_t q_st, int64_t q_sh, int64_t kv_sb,
+                           int64_t kv_st, int64_t kv_sh, int64_t out_sb, int64_t out_st, const void* q,
+                           const void* k, const void* v, const void* out);
+int launch_prefill_f32(const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh, const void* k, const void* v,
+                       int64_t kv_sb, int64_t kv_st, int64_t kv_sh, const int32_t* sel, const int32_t* n_sel,
+                       int64_t cap, int64_t B, int64_t T, int64_t Hq, int64_t Hkv, int64_t bs, int causal,
+                       float scale, void* out, int64_t out_sb, int64_t out_st, hipStream_t stream);
+
 int launch_prefill(const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh, const void* k,
                    const void* v, int64_t kv_sb, int64_t kv_st, int64_t kv_sh, int dtype,
                    const int32_t* sel, const int32_t* n_sel, int64_t cap, int64_t B, int64_t T,

@@ -1,11 +1,12 @@
 // Block-sparse GQA prefill: dispatch and the general VALU kernel.
 //
-// The general kernel covers every supported shape and dtype (fp32 inputs,
+// The general kernel covers every supported shape and dtype (fp32 or bf16,
 // head dims 16..128, any block size, any GQA ratio up to 16). One workgroup
 // serves one (sequence, KV head, query token): it walks the token's selected
 // blocks, stages each block's keys/values of that KV head in LDS once and runs
 // the online softmax for all Hq/Hkv query heads of the group, one wavefront
-// per head. bf16 inputs with D = 64 take the MFMA kernel instead.
+// per head. Inputs with D = 64 take the matrix-core kernels instead (fp32: blocks
+// of 64 or 32 keys).
 #include "common.h"
 #include "kernels.h"
 #include "attend.h"
@@ -347,6 +348,10 @@ int launch_prefill(const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh, cons
                                out_st, q, k, v, out))
         return launch_prefill_mfma(q, q_sb, q_st, q_sh, k, v, kv_sb, kv_st, kv_sh, sel, n_sel, cap,
                                    B, T, Hq, Hkv, bs, causal, scale, out, out_sb, out_st, stream);
+    if (prefill_f32_supported(dtype, T, Hq, Hkv, D, bs, B, sel, q_sb, q_st, q_sh, kv_sb, kv_st, kv_sh, out_sb,
+                              out_st, q, k, v, out))
+        return launch_prefill_f32(q, q_sb, q_st, q_sh, k, v, kv_sb, kv_st, kv_sh, sel, n_sel, cap, B, T, Hq, Hkv, bs,
+                                  causal, scale, out, out_sb, out_st, stream);
     dim3 grid(static_cast<unsigned>(T), static_cast<unsigned>(Hkv), static_cast<unsigned>(B));
     const float sl = scale * kLog2eP;
 #define SPARDA_PF(DT_, DH_)                                                                          \

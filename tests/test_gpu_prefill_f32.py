@@ -1,0 +1,70 @@
+"""The fp32 matrix-core prefill (D = 64): group sizes, ragged tiles and blocks,
+dense and listed, causal and not, against the float64 oracle (max-abs 1e-4, the
+fp32 bar); lists with repeats, and infinite or NaN values of V that a token does
+not attend, against the general kernel (reached through a block size of 16 and
+through the token's own keys)."""
+
+import numpy as np
+import pytest
+import torch
+
+import sparda
+from sparda import synth
+from oracle import sparda_oracle as O
+from helpers import assert_close_out, np32
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("R,T,bs,k,causal,dense", [
+    (1, 33, 64, 8, True, False), (3, 65, 32, 4, True, False), (3, 333, 64, 2, True, False),
+    (4, 200, 32, 4, False, False), (5, 190, 64, 8, True, False), (16, 130, 32, 4, True, False),
+    (3, 127, 64, 8, True, True), (2, 97, 64, 8, False, True), (3, 1, 64, 8, True, True)])
+def test_f32_prefill_against_the_oracle(R, T, bs, k, causal, dense):
+    print(f"[case] f32 R={R} T={T} bs={bs} causal={causal} dense={dense}", flush=True)
+    x = synth.prefill_inputs(2, T, 2 * R, 2, 64, dtype=torch.float32, seed=60 + T)
+    d = {n: t.to(DEV) for n, t in x.items()}
+    sel = n = sel_o = n_o = None
+    if not dense:
+        _, _, sel, n = sparda.route(d["forecast"], sparda.compress(d["k"], bs), bs, k, causal=causal, want_topk=False,
+                                    want_sel=True)
+        sel_o, n_o = sel.cpu().numpy(), n.cpu().numpy()
+    out = sparda.prefill(d["q"], d["k"], d["v"], sel, n, bs, causal=causal)
+    want = O.attention_prefill(np32(x["q"]), np32(x["k"]), np32(x["v"]), sel_o, n_o, bs, causal)
+    assert_close_out(np32(out), want, torch.float32)
+
+
+def test_f32_prefill_repeated_and_out_of_range_entries():
+    # a block of 64 keys listed twice = its four blocks of 16 keys listed twice
+    print("[case] f32 repeats", flush=True)
+    T, Hkv = 260, 2
+    x = synth.prefill_inputs(1, T, 6, Hkv, 64, dtype=torch.float32, seed=4)
+    d = {n: t.to(DEV) for n, t in x.items()}
+    r = np.random.default_rng(5)
+    sel = np.stack([r.integers(-1, 6, (1, Hkv, T)) for _ in range(3)], -1).astype(np.int32)
+    sel[..., 0] = 0
+    sel[..., 2] = np.where(r.random((1, Hkv, T)) < 0.5, sel[..., 1], sel[..., 2])
+    n = r.integers(1, 4, (1, Hkv, T)).astype(np.int32)
+    fine = np.where(sel[..., None] >= 0, 4 * sel[..., None] + np.arange(4), -1).reshape(1, Hkv, T, 12).astype(np.int32)
+    to = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+    got = sparda.prefill(d["q"], d["k"], d["v"], to(sel), to(n), 64)
+    want = sparda.prefill(d["q"], d["k"], d["v"], to(fine), to(4 * n), 16)
+    assert (got - want).abs().max().item() < 1e-5
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_f32_prefill_values_of_unattended_keys_stay_out(bad):
+    print(f"[case] f32 V = {bad}", flush=True)
+    T, at = 150, 70
+    x = synth.prefill_inputs(1, T, 6, 2, 64, dtype=torch.float32, seed=8)
+    v = x["v"].clone()
+    v[0, at, :, 3] = bad
+    q, k = x["q"].to(DEV), x["k"].to(DEV)
+    clean = sparda.prefill(q, k, x["v"].to(DEV), None, None, 64)
+    got = sparda.prefill(q, k, v.to(DEV), None, None, 64)
+    assert (got[:, :at] - clean[:, :at]).abs().max().item() < 1e-5  # tokens before the key: as without it
+    g = got.view(1, T, 6, 64)
+    assert not torch.isfinite(g[:, at:, :, 3]).any()
+    keep = [i for i in range(64) if i != 3]
+    assert (g[..., keep] - clean.view(1, T, 6, 64)[..., keep]).abs().max().item() < 1e-5
