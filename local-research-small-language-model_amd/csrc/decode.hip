@@ -721,82 +721,86 @@ decode_attend_kernel(const void* __restrict__ q, int64_t q_sb, int64_t q_sh,
     __syncthreads();
 }
 
-// The splits of a dense decode (decode_attend_kernel with nsplit > 1): one
-// workgroup per (sequence, KV head) folds the nsplit partials of each of its
-// R heads. Thread (q, e) of Q groups takes the splits q, q + Q, q + 2Q, ...
-// of element e = (head, dim) in split order (32 loads in flight), keeping a
-// running (m, l, o) that is rescaled when a split's maximum exceeds it; the
-// groups are then combined in group order. A split's group depends on its
-// index alone and an empty split (m = -inf, l = 0, o = 0) adds exact zeros,
-// so the splits past the last block (a launch sized for a longer cache)
-// change nothing.
-constexpr int kMergeThreads = 768;
+// The splits of a dense decode (decode_attend_kernel with nsplit > 1, D = 64):
+// one workgroup per (sequence, query head) folds the nsplit partials (m, l, o).
+// Bound by latency (a few hundred 264-byte partials), so every wavefront has its
+// first kMergeU partial rows in flight (lane = dim, coalesced) while the
+// splits' maxima and sums are reduced; the weights exp2(m - M) go through LDS.
+// Wavefront w adds the splits w, w + 4, ... in order and the four sums are added
+// in wavefront order. A split's place in these sums depends on its index alone
+// and an empty split (m = -inf, l = 0, o = 0) adds exact zeros, so the splits
+// past the last block (a launch sized for a longer cache) change nothing.
+constexpr int kMergeWaves = 4;
+constexpr int kMergeThreads = kMergeWaves * kWave;
+constexpr int kMergeU = 32;        // partial rows in flight per wavefront
+constexpr int kMaxSplits = 4096;
 
-template <int DT, int DH>
 __global__ void __launch_bounds__(kMergeThreads)
-decode_merge_kernel(const float* __restrict__ ws_part, int nsplit, int R, int H, int Q, void* __restrict__ out,
+decode_merge_kernel(const float* __restrict__ ws_part, int nsplit, int R, int H, uint16_t* __restrict__ out,
                     int64_t out_sb) {
-    __shared__ float m_q[kMergeThreads], l_q[kMergeThreads], o_q[kMergeThreads];
-    constexpr int U = 32;
-    const int g = blockIdx.x;
+    constexpr int DH = 64;
+    __shared__ float wt[kMaxSplits];
+    __shared__ float red[2][kMergeWaves];
+    __shared__ float o_w[kMergeWaves][DH];
+    const int g = blockIdx.x / R, hh = blockIdx.x % R;
     const int b = blockIdx.y;
-    const int64_t bg = static_cast<int64_t>(b) * H + g;
-    const int RD = R * DH;
-    const int per = static_cast<int>(blockDim.x) / Q;  // elements per round
-    const int t = static_cast<int>(threadIdx.x);
-    const int q = t / per;
-    const int step = R * (DH + 2);
-    for (int e0 = 0; e0 < RD; e0 += per) {  // the same trip count in every thread
-        const int e = e0 + t % per;
-        const bool live = q < Q && e < RD;
-        const int hh = live ? e / DH : 0, d = live ? e % DH : 0;
-        const float* p0 = ws_part + (bg * nsplit * R + hh) * (DH + 2);
-        // this group's splits q + Q j; indices past the last re-read split q
-        // (in bounds) and are not added
-        const int nj = live && q < nsplit ? (nsplit - q + Q - 1) / Q : 0;
-        float M = -__builtin_inff(), num = 0.0f, den = 0.0f;
-        for (int j0 = 0; j0 < nj; j0 += U) {
-            float mv[U], lv[U], ov[U];
+    const int tid = threadIdx.x;
+    const int lane = tid % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int64_t step = static_cast<int64_t>(R) * (DH + 2);
+    const float* p0 = ws_part + ((static_cast<int64_t>(b) * H + g) * nsplit * R + hh) * (DH + 2);
+    // rows past the last split re-read it and are not added
+    float ov[kMergeU];
+    auto fetch = [&](int j0) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int off = (q + Q * (j0 + u < nj ? j0 + u : 0)) * step;
-                mv[u] = p0[off];
-                lv[u] = p0[off + 1];
-                ov[u] = p0[off + 2 + d];
-            }
+        for (int u = 0; u < kMergeU; ++u) {
+            const int i = wave + kMergeWaves * (j0 + u);
+            ov[u] = p0[(i < nsplit ? i : nsplit - 1) * step + 2 + lane];
+        }
+    };
+    // maxima, then weights and the weighted row sums
+    const float l0 = p0[(tid < nsplit ? tid : 0) * step + 1];  // the thread's first split's row sum, with its maximum
+    float M = -__builtin_inff();
+    for (int i = tid; i < nsplit; i += kMergeThreads) {
+        const float m = p0[i * step];
+        wt[i] = m;
+        M = fmaxf(M, m);
+    }
+    fetch(0);
+    M = wave_max(M);
+    if (lane == 0) red[0][wave] = M;
+    __syncthreads();
+    M = red[0][0];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (j0 + u < nj && mv[u] != -__builtin_inff()) {
-                    if (mv[u] > M) {
-                        const float sc = __builtin_amdgcn_exp2f(M - mv[u]);
-                        num = num * sc;
-                        den = den * sc;
-                        M = mv[u];
-                    }
-                    const float wt = __builtin_amdgcn_exp2f(mv[u] - M);
-                    den = den + wt * lv[u];
-                    num = num + wt * ov[u];
-                }
-            }
+    for (int w = 1; w < kMergeWaves; ++w) M = fmaxf(M, red[0][w]);
+    float den = 0.0f;
+    for (int i = tid; i < nsplit; i += kMergeThreads) {
+        const float m = wt[i];
+        const float x = m == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(m - M);
+        wt[i] = x;
+        den = den + x * (i == tid ? l0 : p0[i * step + 1]);
+    }
+    den = wave_sum(den);
+    if (lane == 0) red[1][wave] = den;
+    __syncthreads();
+    float num = 0.0f;
+    const int nj = (nsplit - wave + kMergeWaves - 1) / kMergeWaves;  // this wavefront's splits
+    for (int j0 = 0; j0 < nj; j0 += kMergeU) {
+        if (j0 > 0) fetch(j0);
+#pragma unroll
+        for (int u = 0; u < kMergeU; ++u)
+            if (j0 + u < nj) num = num + wt[wave + kMergeWaves * (j0 + u)] * ov[u];
+    }
+    o_w[wave][lane] = num;
+    __syncthreads();
+    if (wave == 0) {
+        float n_all = 0.0f, d_all = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kMergeWaves; ++w) {
+            n_all = n_all + o_w[w][lane];
+            d_all = d_all + red[1][w];
         }
-        m_q[t] = M;
-        l_q[t] = den;
-        o_q[t] = num;
-        __syncthreads();
-        if (live && q == 0) {
-            float Mall = -__builtin_inff();
-            for (int r = 0; r < Q; ++r) Mall = fmaxf(Mall, m_q[r * per + t]);
-            float n_all = 0.0f, d_all = 0.0f;
-            for (int r = 0; r < Q; ++r) {
-                const float mr = m_q[r * per + t];
-                if (mr == -__builtin_inff()) continue;  // a group without a block
-                const float wt = __builtin_amdgcn_exp2f(mr - Mall);
-                n_all = n_all + wt * o_q[r * per + t];
-                d_all = d_all + wt * l_q[r * per + t];
-            }
-            store_elem<DT>(out, b * out_sb + static_cast<int64_t>(g * R + hh) * DH + d, n_all / d_all);
-        }
-        __syncthreads();  // m_q, l_q, o_q are rewritten by the next round
+        out[b * out_sb + static_cast<int64_t>(g * R + hh) * DH + lane] = f32_to_bf16(n_all / d_all);
     }
 }
 
@@ -827,7 +831,6 @@ struct AttendArgs {
 // block, and with it the result, depends on the length alone, not on the
 // capacity a launch is sized for; no split below two.
 constexpr int64_t kSplitBlocks = 4;
-constexpr int64_t kMaxSplits = 4096;
 
 struct DenseSplit {
     int n = 1;       // splits per (sequence, KV head)
@@ -840,7 +843,7 @@ static int64_t dense_split_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t D) 
 
 static DenseSplit dense_split(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t NB, size_t ws_bytes) {
     int64_t fit = static_cast<int64_t>(ws_bytes) / dense_split_bytes(B, Hq, Hkv, D);
-    fit = fit < kMaxSplits ? fit : kMaxSplits;
+    fit = fit < kMaxSplits ? fit : static_cast<int64_t>(kMaxSplits);
     if (fit < 2) return DenseSplit{};
     int64_t per = kSplitBlocks;
     if (cdiv(NB, per) > fit) per = cdiv(NB, fit);
@@ -909,14 +912,10 @@ static int launch_attend(const AttendArgs& a, hipStream_t stream) {
                            a.new_sb, a.new_sh, a.sel_out, a.n_sel_out, a.out, a.out_sb, a.pos_dev, a.sums, \
                            a.nb_stride, a.update_sums, a.fsel, a.fsel_bf16, a.fs_sb, a.fs_sh, a.absolute,       \
                            a.fscale, pow2, pf, nsplit, split.blocks, a.ws_part);                               \
-        if (nsplit > 1) {                                                                                \
-            const int rd = static_cast<int>(R) * DH_;                                                    \
-            const int qg = rd >= kMergeThreads ? 1 : (kMergeThreads / rd < 4 ? kMergeThreads / rd : 4);  \
-            const int thr = rd >= kMergeThreads ? kMergeThreads : rd * qg;                               \
-            hipLaunchKernelGGL((decode_merge_kernel<DT_, DH_>), dim3(static_cast<unsigned>(a.Hkv),       \
-                               static_cast<unsigned>(a.B)), dim3(thr), 0, stream, a.ws_part, nsplit,     \
-                               static_cast<int>(R), Hkv_i, qg, a.out, a.out_sb);                         \
-        }                                                                                                \
+        if (nsplit > 1)  /* bf16, D = 64 */                                                              \
+            hipLaunchKernelGGL(decode_merge_kernel, dim3(static_cast<unsigned>(a.Hq), static_cast<unsigned>(a.B)), \
+                               dim3(kMergeThreads), 0, stream, a.ws_part, nsplit, static_cast<int>(R), Hkv_i, \
+                               static_cast<uint16_t*>(a.out), a.out_sb);                                 \
     } while (0)
 #define SPARDA_ATT_C(DT_, DH_)                            \
     if (NB <= 256) SPARDA_ATT(DT_, DH_, 4);               \
