@@ -780,6 +780,7 @@ decode_merge_kernel(const float* __restrict__ ws_part, int nsplit, int R, int H,
         wt[i] = x;
         den = den + x * (i == tid ? l0 : p0[i * step + 1]);
     }
+    asm volatile("s_nop 1" : "+v"(den));  // the wait states of the reduction's first DPP, on every way out of the loop
     den = wave_sum(den);
     if (lane == 0) red[1][wave] = den;
     __syncthreads();
