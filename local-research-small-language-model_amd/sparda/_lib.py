@@ -164,9 +164,40 @@ def load() -> ctypes.CDLL:
 
 def call(name: str, *args) -> None:
     """Call an entry point and turn a non-zero status into an exception."""
-    lib = load()
-    rc = getattr(lib, name)(*args)
+    rc = getattr(_lib or load(), name)(*args)
     if rc != 0:
-        msg = (lib.sparda_last_error() or b"").decode(errors="replace")
-        cls = SpardaArgumentError if rc < 0 else SpardaError
-        raise cls(name, rc, msg)
+        fail(name, rc)
+
+
+def fail(name: str, rc: int) -> None:
+    """Raise the exception of a non-zero status of entry point `name`."""
+    msg = (load().sparda_last_error() or b"").decode(errors="replace")
+    cls = SpardaArgumentError if rc < 0 else SpardaError
+    raise cls(name, rc, msg)
+
+
+# entry points the native host path calls, in the order of its table
+_HOST_ENTRIES = ("compress", "route", "prefill", "prefill_routed", "prefill_chunked", "decode",
+                 "decode_workspace_bytes", "decode_selected", "decode_dense_workspace_bytes", "decode_sums", "produce",
+                 "produce_at", "produce_cache_at", "ffn_decode", "rows_residual", "norm_gemv", "teacher_mass")
+
+
+class _NoHost:
+    """Without the extension module every operator takes its Python path."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def load_host():
+    """The native host path (sparda._host) bound to the loaded library."""
+    try:
+        from . import _host
+    except ImportError:
+        return _NoHost()
+    import torch
+
+    lib = load()
+    _host.bind(torch._C._cuda_getCurrentRawStream,
+               tuple(ctypes.cast(getattr(lib, "sparda_" + n), ctypes.c_void_p).value for n in _HOST_ENTRIES))
+    return _host

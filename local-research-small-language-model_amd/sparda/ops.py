@@ -26,6 +26,20 @@ def _dtype_code(t: torch.Tensor) -> int:
         raise TypeError(f"sparda: unsupported dtype {t.dtype} (float32 or bfloat16)") from None
 
 
+class _LazyHost:
+    """The native host path, bound at its first use. Its functions take an
+    operator's call in the common form and return the result, an int status to
+    raise, or None: the operator then goes on with its own full path."""
+
+    def __getattr__(self, name):
+        global _host
+        _host = _lib.load_host()
+        return getattr(_host, name)
+
+
+_host = _LazyHost()
+
+
 def require_device(*tensors: Optional[torch.Tensor]) -> torch.device:
     dev = None
     for t in tensors:
@@ -69,6 +83,9 @@ def default_scale(dim: int) -> float:
 
 def compress(k: torch.Tensor, block_size: int) -> torch.Tensor:
     """k [B,S,H,D] (fp32/bf16) -> prototypes [B,NB,H,D] fp32 (model/forecast.py:57-78)."""
+    r = _host.compress(k, block_size)
+    if r is not None:
+        return r if type(r) is not int else _lib.fail("sparda_compress", r)
     dev = require_device(k)
     _inference_only(k)
     k = _rowmajor(k)
@@ -91,6 +108,10 @@ def route(forecast: torch.Tensor, protos: torch.Tensor, block_size: int, top_k: 
     Returns (topk int32 [B,H,Tq,ke] | None, scores fp32 [B,H,Tq,NB] | None,
     sel int32 [B,H,Tq,cap] | None, n_sel int32 [B,H,Tq] | None).
     """
+    if want_topk and not (want_scores or want_sel):
+        r = _host.route(forecast, protos, block_size, top_k, causal, score_pos0, query_pos0, scale)
+        if r is not None:
+            return (r, None, None, None) if type(r) is not int else _lib.fail("sparda_route", r)
     dev = require_device(forecast, protos)
     _inference_only(forecast)
     forecast = _rowmajor(forecast)
@@ -213,6 +234,10 @@ def prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sel: Optional[tor
     ``select_fixed`` ([B,Hkv,T,cap] / [B,Hkv,T]) or None for dense.
     Returns out [B,T,Hq*D] in q's dtype.
     """
+    if sel is None and out is None:
+        r = _host.prefill(q, k, v, block_size, causal, scale)
+        if r is not None:
+            return r if type(r) is not int else _lib.fail("sparda_prefill", r)
     dev = require_device(q, k, v, sel, n_sel)
     _inference_only(q, k, v)
     if not (q.dtype == k.dtype == v.dtype):
@@ -274,6 +299,10 @@ def prefill_routed(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, forecast: 
     with want_sel (the lists ``route`` returns with want_sel and the same
     sel_cap, default min(top_k, NB) + 2).
     """
+    if not want_sel and out is None:
+        r = _host.prefill_routed(q, k, v, forecast, protos, block_size, top_k, causal, scale, route_scale)
+        if r is not None:
+            return r if type(r) is not int else _lib.fail("sparda_prefill_routed", r)
     dev = require_device(q, k, v, forecast, protos)
     _inference_only(q, k, v, forecast)
     if not (q.dtype == k.dtype == v.dtype):
@@ -339,6 +368,10 @@ def prefill_chunked(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, topk: Opt
     in one launch where the shape allows. q [B,T,Hq,D], k/v [B,T,Hkv,D].
     Returns out [B,T,Hq*D], or (out, sel, n_sel) with want_sel (the lists
     ``select_chunked`` returns)."""
+    if not want_sel and out is None:
+        r = _host.prefill_chunked(q, k, v, topk, block_size, top_k, scale)
+        if r is not None:
+            return r if type(r) is not int else _lib.fail("sparda_prefill_chunked", r)
     dev = require_device(q, k, v, topk)
     _inference_only(q, k, v)
     if not (q.dtype == k.dtype == v.dtype):
@@ -486,6 +519,11 @@ def decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, S: int
     forecast [B,Hkv,Df] or None; routing "reference" | "absolute".
     Returns out [B,Hq*D], or (out, extras) when want_protos / want_sel.
     """
+    if workspace is not None and workspace.buf is not None and protos_in is None and out is None and not (
+            want_protos or want_sel) and routing in ("reference", "absolute"):
+        r = _host.decode(q, k_cache, v_cache, S, forecast, block_size, top_k, routing == "absolute", scale, workspace.buf)
+        if r is not None:
+            return r if type(r) is not int else _lib.fail("sparda_decode", r)
     dev = require_device(q, k_cache, v_cache, forecast, protos_in)
     _inference_only(q, k_cache, v_cache)
     if not (q.dtype == k_cache.dtype == v_cache.dtype):
@@ -548,6 +586,10 @@ def decode_selected(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, S: int, b
     sel[b,g,i]. sel=None: dense over [0, S). k_new/v_new [B,Hkv,D]: the key and
     value of position S-1 (overriding what k/v hold there).
     """
+    if sel is None and out is None and k_new is None and v_new is None and not compact:
+        r = _host.decode_dense(q, k, v, S, block_size, scale)
+        if r is not None:
+            return r if type(r) is not int else _lib.fail("sparda_decode_selected", r)
     dev = require_device(q, k, v, sel, n_sel, k_new, v_new)
     _inference_only(q, k, v, k_new, v_new)
     if not (q.dtype == k.dtype == v.dtype):
@@ -605,6 +647,9 @@ def teacher_block_mass(q: torch.Tensor, k: torch.Tensor, block_size: int = 64, c
     query heads of each KV head (model/forecast.py:141-193, steps 1-3), from
     q [B,T,Hq,64] and k [B,T,Hkv,64] bf16 without materialising the weights.
     Returns [B,Hkv,T,ceil(T/64)] fp32."""
+    r = _host.teacher_mass(q, k, block_size, causal, scale)
+    if r is not None:
+        return r if type(r) is not int else _lib.fail("sparda_teacher_mass", r)
     dev = require_device(q, k)
     _inference_only(q, k)
     q, k = _rowmajor(q), _rowmajor(k)
@@ -643,6 +688,11 @@ def produce(x: torch.Tensor, w_stacked: torch.Tensor, n_q: int, n_kv: int, n_f: 
     the new keys and values as rows *pos_dev + t (the cache append of
     KVCache.update, model/attention/base.py:19-29; decode-sized batches,
     B*T <= 16); block sums are then the decode launch's to update."""
+    if f_dtype is torch.bfloat16 or f_dtype is torch.float32:
+        r = _host.produce(x, w_stacked, n_q, n_kv, n_f, eps, rope_cos, rope_sin, pos0, f_dtype is torch.float32, pos_dev,
+                          k_cache, v_cache)
+        if r is not None:
+            return r if type(r) is not int else _lib.fail("sparda_produce", r)
     dev = require_device(x, w_stacked, rope_cos, rope_sin, pos_dev)
     _inference_only(x, w_stacked)
     if x.dtype != torch.bfloat16 or w_stacked.dtype != torch.bfloat16:
@@ -707,6 +757,11 @@ def decode_sums(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, S: int, forec
     recomputed from its rows (as block_sums(k, cb*bs, S - cb*bs, ...) does)
     and stored, so the caller needs no separate sums update after appending.
     Returns out [B,Hq*D], or (out, sel, n_sel) with want_sel."""
+    if out is None and not want_sel and routing in ("reference", "absolute"):
+        r = _host.decode_sums(q, k, v, S, forecast, block_sums, block_size, top_k, routing == "absolute", pos_dev, scale,
+                              update_current)
+        if r is not None:
+            return r if type(r) is not int else _lib.fail("sparda_decode_sums", r)
     dev = require_device(q, k, v, forecast, block_sums, pos_dev)
     _inference_only(q, k, v)
     if not (q.dtype == k.dtype == v.dtype):
@@ -761,6 +816,10 @@ def ffn_decode(x: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, e
     layer's prefetch copy carried by the two launches (sparda_ffn_decode_prefetch),
     each a decode_at prefetch spec with ``stage`` 2 and ``parts`` / ``part``,
     at position pos_dev over arenas of block_size-key blocks."""
+    if prefetch is None and out is None:
+        r = _host.ffn_decode(x, w_gate_up, w_down, eps)
+        if r is not None:
+            return r if type(r) is not int else _lib.fail("sparda_ffn_decode", r)
     dev = require_device(x, w_gate_up, w_down, out)
     _inference_only(x, w_gate_up, w_down)
     if not (x.dtype == w_gate_up.dtype == w_down.dtype == torch.bfloat16):
@@ -808,6 +867,10 @@ def rows_residual(a: torch.Tensor, w: torch.Tensor, res: torch.Tensor,
     model/attention/sparse.py:183). a [B,T,K], w [N,K], res [B,T,N], all bf16,
     B*T <= 16. The projection is rounded to bf16 before the sum, as the
     unfused pair does. Returns [B,T,N] bf16."""
+    if out is None:
+        r = _host.rows_residual(a, w, res)
+        if r is not None:
+            return r if type(r) is not int else _lib.fail("sparda_rows_residual", r)
     dev = require_device(a, w, res, out)
     _inference_only(a, w, res)
     if not (a.dtype == w.dtype == res.dtype == torch.bfloat16):
@@ -837,6 +900,10 @@ def norm_gemv(x: torch.Tensor, w_folded: torch.Tensor, eps: float,
     last RMSNorm and its tied output projection, model/model.py:79-157 with
     model/norm.py:15-21): x [B,T,C] bf16 with B*T <= 16, w_folded [N,C] bf16 =
     W * norm_weight (folded into the columns). Returns [B,T,N] bf16."""
+    if out is None:
+        r = _host.norm_gemv(x, w_folded, eps)
+        if r is not None:
+            return r if type(r) is not int else _lib.fail("sparda_norm_gemv", r)
     dev = require_device(x, w_folded, out)
     _inference_only(x, w_folded)
     if not (x.dtype == w_folded.dtype == torch.bfloat16):
