@@ -2,8 +2,8 @@
 // BS = 64 or 32 keys, at most 10 selected blocks per token).
 //
 // One workgroup of 12 wavefronts (one per CU, three per SIMD) serves one
-// (sequence b, KV head g, query window qb): W = 128 query tokens (64 for
-// R = 4, whose 128-token accumulators would not fit the LDS) x R = Hq/Hkv
+// (sequence b, KV head g, query window qb): W query tokens (16 to 128, chosen
+// by pick_window) x R = Hq/Hkv
 // query heads = W*R columns, column c = token * R + head. Every query token picks its own blocks, so a KV block
 // is attended by only some of the window's columns. For each block j in the
 // union of the window's selections, the columns that selected j are packed,
@@ -51,36 +51,37 @@ constexpr int kCMaxNB = 1024;                   // KV blocks
 // wavefronts per workgroup: one workgroup per CU, three wavefronts per SIMD
 constexpr int kCWaves = 12;
 constexpr int kCThreads = kCWaves * kWave;
+constexpr int64_t kCCus = 256;                  // compute units: one workgroup each
 
-// a query window of W tokens (128; 64 for R = 4, whose accumulators for 128
-// tokens would not fit the LDS) per workgroup. Its 64-token sets are routed
-// by kSetWaves waves each, whose first wave then holds the set's tokens
-// (lane = token) through the set-up.
+// a query window of W tokens per workgroup (pick_window chooses W). Each of its
+// 64-token sets (one set of W tokens below 64) is held by one of every
+// kSetWaves waves (lane = token) through the set-up.
 template <int W>
 struct Win {
-    static_assert(W == 64 || W == 128, "windows of 64 or 128 tokens");
+    static_assert(W == 16 || W == 32 || W == 64 || W == 128, "windows of 16 to 128 tokens");
+    static constexpr int kSets = W < 64 ? 1 : W / 64;
     static constexpr int kMaxPairs = W * kCMaxCap;               // (token, block) pairs of a window
     static constexpr int kMaxUnion = kMaxPairs < kCMaxNB ? kMaxPairs : kCMaxNB;  // distinct blocks
-    static constexpr int kSetWaves = kCWaves / (W / 64);
+    static constexpr int kSetWaves = kCWaves / kSets;
 };
 
 // the tokens of a window that selected a block: bit t of word t / 64
 template <int W>
 struct TokMask {
-    unsigned long long w[W / 64];
+    unsigned long long w[Win<W>::kSets];
 };
 template <int W>
 __device__ __forceinline__ bool mask_any(const TokMask<W>& m) {
     bool a = false;
 #pragma unroll
-    for (int i = 0; i < W / 64; ++i) a = a || m.w[i] != 0ull;
+    for (int i = 0; i < Win<W>::kSets; ++i) a = a || m.w[i] != 0ull;
     return a;
 }
 template <int W>
 __device__ __forceinline__ int mask_count(const TokMask<W>& m) {
     int n = 0;
 #pragma unroll
-    for (int i = 0; i < W / 64; ++i) n += __popcll(m.w[i]);
+    for (int i = 0; i < Win<W>::kSets; ++i) n += __popcll(m.w[i]);
     return n;
 }
 // selecting tokens before token t
@@ -88,7 +89,7 @@ template <int W>
 __device__ __forceinline__ int mask_count_below(const TokMask<W>& m, int t) {
     int n = 0;
 #pragma unroll
-    for (int i = 0; i < W / 64; ++i) {
+    for (int i = 0; i < Win<W>::kSets; ++i) {
         const int lo = 64 * i;
         n += t >= lo + 64 ? __popcll(m.w[i]) : (t > lo ? __popcll(m.w[i] & ((1ull << (t - lo)) - 1ull)) : 0);
     }
@@ -108,8 +109,10 @@ struct CompactSmem {
     static constexpr int kMaxItems = (R * Win<W>::kMaxPairs) / 16 + kMaxUnion;
     // fp32 accumulators, slab layout: acc[s * kCols + col] = O[col][4s .. 4s+3].
     // During the set-up the same bytes hold the per-block token bitmaps, the
-    // block -> union map and per-token facts.
-    float4 acc[16 * kCols];
+    // block -> union map and per-token facts (more than the accumulators of a
+    // narrow window).
+    static constexpr int kSetup = (kCMaxNB * static_cast<int>(sizeof(TokMask<W>) + sizeof(uint16_t)) + 15) / 16;
+    float4 acc[16 * kCols > kSetup ? 16 * kCols : kSetup];
     uint16_t vstage[kCWaves][32 * 64];          // half a V block per wave, swizzled
     uint32_t items[kMaxItems];                  // u | first tile << 16
     float mref[kCols];                          // log2 units
@@ -134,12 +137,10 @@ __device__ __forceinline__ float key_to_float(uint32_t k) {
 
 }  // namespace
 
-// W = 128 (R <= 3) or 64 (R = 4): one workgroup of 12 wavefronts per CU; the
-// wider window's tiles are fuller when each token's selections are spread
-// over many blocks.
+// W: tokens per window (pick_window); one workgroup of 12 wavefronts per CU.
 // BS: keys per KV block (64 or 32).
 // FDT < 0: the token lists come from sel / n_sel. FDT = the forecast's dtype:
-// the kernel routes its own window first (the router's per-set code, so the
+// the kernel routes its own window first (the router's code, so the
 // lists are the router's bit for bit) and, with rt.sel set, also writes them
 // out as the router does.
 template <int R, int BS, int FDT, int W>
@@ -205,17 +206,43 @@ prefill_compact_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_s
     // blocks past the token's own (no key of theirs is allowed) are dropped
     const int tlim = static_cast<int>(causal ? (t0 + tok) / BS : NB - 1);
     if constexpr (FDT >= 0) {
-        // each group of kSetWaves waves routes 64 of the window's tokens,
-        // every wave scoring its share of the candidate blocks; the group's
-        // first wave merges (through the group's V staging bytes, unused
-        // until the tiles: 4 KB per wave, one wave's key lists) and holds
-        // token tok's picks
-        int32_t picks[kCRouteK];
-        if (route_set<FDT, kCRouteDf, kCRouteK, kSetWaves>(
-                rt.f, rt.fsb, rt.fst, rt.fsh, rt.protos, b, g, H, qb * (W / 64) + wave / kSetWaves, T, NB, BS,
-                rt.ke, causal, 0, rt.scale, nullptr, 0,
-                reinterpret_cast<double*>(&sm.vstage[kSetWaves * (wave / kSetWaves)][0]), picks) &&
-            tok < t_valid) {
+        // the window's rows in parts of 16 RT, each scored by kRG wavefronts that
+        // share the candidate blocks; the parts' lists are merged by the owner
+        // waves, token tok in lane tok % 64 (all of it in the V staging bytes,
+        // unused until the tiles)
+        constexpr int kRT = W == 128 ? 2 : 1, kRP = W / 16 / kRT, kRG = 3;
+        using Shape = RouteShape<kCRouteDf, kCWaves, kRP, kRG, kRT, 1>;
+        static_assert(Shape::kFloats * sizeof(float) <= sizeof(sm.vstage) &&
+                          kRG * kCRouteK * W * sizeof(double) <= sizeof(sm.vstage),
+                      "routing in the V staging bytes");
+        KeyTopK<kCRouteK> best[kRT];
+        route_tiles<FDT, kCRouteDf, kCRouteK, kCWaves, kRP, kRG, kRT, 1>(
+            rt.f, rt.fsb, rt.fst, rt.fsh, rt.protos, b, g, H, t0, W, T, NB, BS, causal, 0, rt.scale, nullptr,
+            reinterpret_cast<float*>(&sm.vstage[0][0]), best);
+        __syncthreads();  // the last prototypes have been read
+        double* lists = reinterpret_cast<double*>(&sm.vstage[0][0]);  // [kRG][kCRouteK][W]
+        if (wave < kRP * kRG) {
+#pragma unroll
+            for (int i = 0; i < kRT; ++i)
+#pragma unroll
+                for (int e = 0; e < kCRouteK; ++e)
+                    if (e % 4 == grp)  // the four lanes of a row hold the same list
+                        lists[((wave / kRP) * kCRouteK + e) * W + 16 * (kRT * (wave % kRP) + i) + col16] = best[i].r[e];
+        }
+        __syncthreads();
+        if (has_tok) {
+            KeyTopK<kCRouteK> row;
+#pragma unroll
+            for (int e = 0; e < kCRouteK; ++e) row.r[e] = lists[e * W + tok];
+#pragma unroll
+            for (int o = 1; o < kRG; ++o) {
+                double other[kCRouteK];
+#pragma unroll
+                for (int e = 0; e < kCRouteK; ++e) other[e] = lists[(o * kCRouteK + e) * W + tok];
+                row.merge(other);
+            }
+            int32_t picks[kCRouteK];
+            route_picks(row, rt.ke, picks);
             // {0, own} U picks, own = the token's block (prefill positions start at 0)
             const int own = static_cast<int>((t0 + tok) / BS);
             int raw[kCMaxCap];
@@ -274,7 +301,7 @@ prefill_compact_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_s
     // the first key of the token's first listed block (always an allowed key),
     // or -1: its score is the column's reference (set-up 2). Held in the row
     // sums' bytes until set-up 3 clears them.
-    if (owner) reinterpret_cast<int*>(sm.lsum)[tok] = (has_tok && lst[0] != kSentinel) ? lst[0] * BS : -1;
+    if (owner && tok < W) reinterpret_cast<int*>(sm.lsum)[tok] = (has_tok && lst[0] != kSentinel) ? lst[0] * BS : -1;
     for (int i = tid; i <= jmax; i += kT) bitmap[i] = Mask{};
     __syncthreads();
     if (has_tok) {
@@ -737,10 +764,9 @@ static bool compact_layout_ok(int64_t R, int64_t q_sb, int64_t q_st, int64_t q_s
 }
 
 // 128-token windows wherever their LDS fits (R <= 3): twice the tokens of a
-// 64-token window fill the tiles of each selected block. Measured faster at
-// every tested length, with the same output bit for bit (each column's sums do
-// not depend on its tile mates).
-static int pick_window(int64_t R) { return R <= 3 ? 128 : 64; }
+// 64-token window fill the tiles of each selected block. The output is the same
+// bit for bit: a column's sums do not depend on its tile mates.
+static int pick_window(int64_t R, int64_t, int64_t) { return R <= 3 ? 128 : 64; }
 
 // Polls an ordering wait makes before the workgroup abandons it (the window
 // is then NaN and the status word flags it). SPARDA_PREFILL_WAIT_LIMIT
@@ -787,13 +813,15 @@ static int launch_compact(const void* q, int64_t q_sb, int64_t q_st, int64_t q_s
                           int64_t bs, int causal, float scale, void* out, int64_t out_sb, int64_t out_st,
                           hipStream_t stream) {
     const int64_t R = Hq / Hkv;
-    const int W = pick_window(R);  // 128, or 64 for R = 4
+    const int W = pick_window(R, B * Hkv, T);
     const int64_t NBq = cdiv(T, W);  // query windows per (sequence, KV head)
     dim3 grid(static_cast<unsigned>(B * Hkv * NBq));
     const float sl = scale * kCLog2e;
     const uint32_t spin = wait_limit();
 #define SPARDA_PC(R_, W_)                                                                                    \
-    if (bs == 32) SPARDA_PCB(R_, 32, W_); else SPARDA_PCB(R_, 64, W_)
+    do { if (bs == 32) SPARDA_PCB(R_, 32, W_); else SPARDA_PCB(R_, 64, W_); } while (0)
+#define SPARDA_PCW(R_)                                                                                       \
+    if (W == 128) SPARDA_PC(R_, 128); else if (W == 64) SPARDA_PC(R_, 64); else if (W == 32) SPARDA_PC(R_, 32); else SPARDA_PC(R_, 16)
 #define SPARDA_PCB(R_, BS_, W_)                                                                              \
     hipLaunchKernelGGL((prefill_compact_kernel<R_, BS_, FDT, W_>), grid, dim3(kCThreads), 0, stream,          \
                        static_cast<const uint16_t*>(q), q_sb, q_st, q_sh, static_cast<const uint16_t*>(k),    \
@@ -801,11 +829,14 @@ static int launch_compact(const void* q, int64_t q_sb, int64_t q_st, int64_t q_s
                        static_cast<int>(Hkv), NBq, causal, sl, static_cast<uint16_t*>(out), out_sb, out_st, rt, \
                        spin)
     switch (R) {
-        case 1: SPARDA_PC(1, 128); break;
-        case 2: SPARDA_PC(2, 128); break;
-        case 3: SPARDA_PC(3, 128); break;
-        default: SPARDA_PC(4, 64); break;
+        case 1: SPARDA_PCW(1); break;
+        case 2: SPARDA_PCW(2); break;
+        case 3: SPARDA_PCW(3); break;
+        default:
+            if (W == 64) SPARDA_PC(4, 64); else if (W == 32) SPARDA_PC(4, 32); else SPARDA_PC(4, 16);
+            break;
     }
+#undef SPARDA_PCW
 #undef SPARDA_PCB
 #undef SPARDA_PC
     return check_hip(hipGetLastError(), "prefill_compact_kernel");

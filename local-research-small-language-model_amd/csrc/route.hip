@@ -10,6 +10,7 @@
 #include "chunk.h"
 #include "common.h"
 #include "kernels.h"
+#include "mfma.h"
 #include "select.h"
 #include "route_rows.h"
 
@@ -74,20 +75,13 @@ int launch_compress(const void* k, int dtype, int64_t B, int64_t S, int64_t H, i
 }
 
 // ---------------------------------------------------------------------------
-// router: one lane per query row. Under the causal mask a workgroup of
-// kRouteWaves wavefronts takes two sets of 64 consecutive rows of one (b, h):
-// set p and its mirror NS-1-p, so that every workgroup scores about the same
-// number of (row, block) pairs; without it every set has the same work and a
-// workgroup takes one (twice the workgroups, four wavefronts per SIMD instead
-// of two at B=1, T=16384). Within a set the waves split the candidate blocks
-// (wave w scores the blocks j = w mod kRouteWaves), so the block index is
-// uniform across the wavefront: every 16-lane row of the wavefront loads the
-// block's prototype with one coalesced load (lane i of the row holds elements
-// E*i .. E*i+E-1, E = DF/16), one block ahead of its use, and the fma chain
-// takes element d from lane d/E of the row through a DPP row broadcast. Every
-// lane keeps a descending list of route keys; after a set the waves' lists are
-// merged through LDS by one wave (rotating with the set), which writes the
-// rows' outputs.
+// router. Under the causal mask a workgroup of kRouteWaves wavefronts takes two
+// sets of 64 consecutive rows of one (b, h): set p and its mirror NS-1-p, so
+// that every workgroup scores about the same number of (row, block) pairs;
+// without it every set has the same work and a workgroup takes one. Within a
+// set every wavefront takes 16 rows and all candidate blocks, 32 at a time
+// (two independent product chains), staged once in LDS for the four of them
+// (route_tiles); its lanes 0..15 then write their rows' outputs.
 // ---------------------------------------------------------------------------
 template <int FDT, int DF, int KMAX>
 __global__ void __launch_bounds__(kRouteThreads)
@@ -96,8 +90,11 @@ route_rows_kernel(const void* __restrict__ f, int64_t fsb, int64_t fst, int64_t 
                   int ke, int causal, int64_t score_pos0, int64_t query_pos0, float scale,
                   int32_t* __restrict__ topk, float* __restrict__ scores,
                   int32_t* __restrict__ sel, int32_t* __restrict__ n_sel, int cap) {
-    extern __shared__ double lists[];  // [kRouteWaves][KMAX][kWave]
+    using Shape = RouteShape<DF, kRouteWaves, kRouteWaves, 1, 1, 2>;
+    static_assert(Shape::kRows == kWave, "a set is 64 rows");
+    __shared__ __attribute__((aligned(16))) float lds[Shape::kFloats];
     const int lane = threadIdx.x % kWave;
+    const int wave = threadIdx.x / kWave;
     const int h = blockIdx.y;
     const int b = blockIdx.z;
     const int64_t NS = cdiv(Tq, kWave);
@@ -106,13 +103,15 @@ route_rows_kernel(const void* __restrict__ f, int64_t fsb, int64_t fst, int64_t 
     for (int pass = 0; pass < 2; ++pass) {
         const int64_t set = pass == 0 ? pair : NS - 1 - pair;
         if (pass == 1 && (!causal || set == pair)) break;  // one set without the mask; an odd count's middle set
-        const int m = static_cast<int>((2 * pair + pass) % kRouteWaves);
+        KeyTopK<KMAX> best[1];
+        __syncthreads();  // the previous set's last chunk has been read
+        route_tiles<FDT, DF, KMAX, kRouteWaves, kRouteWaves, 1, 1, 2>(f, fsb, fst, fsh, protos, b, h, H, set * kWave,
+                                                                      kWave, Tq, NB, bs, causal, score_pos0, scale,
+                                                                      scores, lds, best);
+        const int64_t t = set * kWave + 16 * wave + lane;
+        if (lane >= 16 || t >= Tq) continue;
         int32_t picks[KMAX];
-        if (!route_set<FDT, DF, KMAX>(f, fsb, fst, fsh, protos, b, h, H, set, Tq, NB, bs, ke, causal, score_pos0,
-                                      scale, scores, m, lists, picks))
-            continue;
-        const int64_t t = set * kWave + lane;
-        if (t >= Tq) continue;
+        route_picks(best[0], ke, picks);
         const int64_t row = (static_cast<int64_t>(b) * H + h) * Tq + t;
         if (topk) {
             int32_t* tr = topk + row * ke;
@@ -142,8 +141,7 @@ static int launch_route_df(const void* f, int64_t fsb, int64_t fst, int64_t fsh,
     const int64_t pairs = causal ? cdiv(cdiv(Tq, kWave), 2) : cdiv(Tq, kWave);
     dim3 grid(static_cast<unsigned>(pairs), static_cast<unsigned>(H), static_cast<unsigned>(B));
 #define SPARDA_ROUTE(KM_)                                                                          \
-    hipLaunchKernelGGL((route_rows_kernel<FDT, DF, KM_>), grid, dim3(kRouteThreads),               \
-                       static_cast<size_t>(kRouteWaves) * KM_ * kWave * sizeof(double), stream,    \
+    hipLaunchKernelGGL((route_rows_kernel<FDT, DF, KM_>), grid, dim3(kRouteThreads), 0, stream,    \
                        f, fsb, fst, fsh, protos, Tq, static_cast<int>(H), NB,                      \
                        static_cast<int>(bs), ke, causal, score_pos0, query_pos0, scale,            \
                        topk, scores, sel, n_sel, cap)

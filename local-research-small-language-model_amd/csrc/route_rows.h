@@ -1,11 +1,11 @@
-// One set of 64 consecutive query rows routed by a group of wavefronts of
-// one workgroup (lane = row): forecast x prototype scores (the
-// canonical fma chain), the per-row top-k of route keys, merged across the
-// waves. Shared by the stand-alone router and the prefill kernel that routes
+// Rows of (sequence, head) routed by a workgroup: forecast x prototype scores
+// (the canonical fma chain, on the matrix cores) and the per-row top-k of route
+// keys. Shared by the stand-alone router and the prefill kernel that routes
 // its own query window, so both produce the same picks bit for bit.
 #pragma once
 
 #include "common.h"
+#include "mfma.h"
 #include "select.h"
 
 namespace sparda {
@@ -13,212 +13,227 @@ namespace sparda {
 constexpr int kRouteWaves = 4;
 constexpr int kRouteThreads = kRouteWaves * kWave;
 
-// N consecutive fp32 values (N in {1, 2, 4, 8}), 4*N-byte aligned
-template <int N>
-__device__ __forceinline__ void load_f32(const float* __restrict__ p, float (&o)[N]) {
-    if constexpr (N == 1) {
-        o[0] = p[0];
-    } else if constexpr (N == 2) {
-        const float2 v = *reinterpret_cast<const float2*>(p);
-        o[0] = v.x; o[1] = v.y;
-    } else {
+// top-k lists of lanes whose 16-lane rows differ in bit 0 (SWAP 16) or bit 1
+// (32) of their row index, merged into both
+template <int SWAP, int KMAX>
+__device__ __forceinline__ void merge_rows(KeyTopK<KMAX>& best) {
+    double a[KMAX], c[KMAX];
 #pragma unroll
-        for (int q = 0; q < N; q += 4) {
-            const float4 v = *reinterpret_cast<const float4*>(p + q);
-            o[q] = v.x; o[q + 1] = v.y; o[q + 2] = v.z; o[q + 3] = v.w;
-        }
-    }
-}
-
-// Two fma chains, one step: acc[c] = fma(a, element of lane I of this lane's
-// 16-lane row of p[c], acc[c]), each a v_fmac_f32 with a DPP row_newbcast
-// source (a separate DPP move does not fold into the fma, which is a VOP3 op
-// at that point). A DPP instruction needs two wait states after a VALU write
-// of any register it reads. The compiler does not track that for inline
-// assembly, so the steps carry their own: the two fmas of a step write
-// different accumulators and end with s_nop 0, so an accumulator is read two
-// wait states after its last write, and the steps that first read the
-// prototype registers (FIRST) start with s_nop 1. What the compiler places
-// between steps (spill reloads, copies) is checked on the built code by the
-// test suite. (Four chains without the s_nop measured no faster: the nop
-// costs the wave an issue cycle, not the SIMD, whose other wave issues.)
-template <int I, bool FIRST>
-__device__ __forceinline__ void fma_row_bcast(float (&acc)[2], float a, const float (&p)[2]) {
-    if constexpr (FIRST)
-        asm("s_nop 1\n\tv_fmac_f32_dpp %0, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f32_dpp %1, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\ts_nop 0"
-            : "+v"(acc[0]), "+v"(acc[1]) : "v"(p[0]), "v"(p[1]), "v"(a), "n"(I));
-    else
-        asm("v_fmac_f32_dpp %0, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f32_dpp %1, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\ts_nop 0"
-            : "+v"(acc[0]), "+v"(acc[1]) : "v"(p[0]), "v"(p[1]), "v"(a), "n"(I));
-}
-// acc[c] = fma chain over d = E*I + e (I = I0..15, e = 0..E-1) with element d
-// of prototype c taken from lane I of the row (register pc[e][c])
-template <int E, int DF, int C, int I0 = 0>
-__device__ __forceinline__ void row_fma_chains(const float (&fr)[DF], const float (&pc)[E][C],
-                                               float (&acc)[C]) {
-    if constexpr (I0 < 16) {
-#pragma unroll
-        for (int e = 0; e < E; ++e) fma_row_bcast<I0, I0 == 0>(acc, fr[E * I0 + e], pc[e]);
-        row_fma_chains<E, DF, C, I0 + 1>(fr, pc, acc);
-    }
-}
-
-// The DF forecast elements at element offset `base` as fp32: 16-byte vector
-// loads where every row is 16-byte aligned (vec, uniform), else one element
-// at a time.
-template <int FDT, int DF>
-__device__ __forceinline__ void load_forecast_row(const void* __restrict__ f, int64_t base, bool vec,
-                                                  float (&fr)[DF]) {
-    if (vec) {
-        if constexpr (FDT == SPARDA_F32) {
-            const float4* src = reinterpret_cast<const float4*>(static_cast<const float*>(f) + base);
-#pragma unroll
-            for (int q = 0; q < DF / 4; ++q) {
-                const float4 w = src[q];
-                fr[4 * q] = w.x; fr[4 * q + 1] = w.y; fr[4 * q + 2] = w.z; fr[4 * q + 3] = w.w;
-            }
+    for (int i = 0; i < KMAX; ++i) {
+        const uint32_t lo = static_cast<uint32_t>(__double2loint(best.r[i]));
+        const uint32_t hi = static_cast<uint32_t>(__double2hiint(best.r[i]));
+        if constexpr (SWAP == 16) {
+            const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+            const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+            a[i] = __hiloint2double(static_cast<int>(h[0]), static_cast<int>(l[0]));
+            c[i] = __hiloint2double(static_cast<int>(h[1]), static_cast<int>(l[1]));
         } else {
-            const uint4* src = reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(f) + base);
-#pragma unroll
-            for (int q = 0; q < DF / 8; ++q) {
-                const uint4 w = src[q];
-                const uint32_t u[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    fr[8 * q + 2 * e] = __uint_as_float(u[e] << 16);
-                    fr[8 * q + 2 * e + 1] = __uint_as_float(u[e] & 0xffff0000u);
-                }
-            }
+            const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+            const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+            a[i] = __hiloint2double(static_cast<int>(h[0]), static_cast<int>(l[0]));
+            c[i] = __hiloint2double(static_cast<int>(h[1]), static_cast<int>(l[1]));
         }
-    } else {
-#pragma unroll
-        for (int d = 0; d < DF; ++d) fr[d] = load_elem<FDT>(f, base + d);
     }
+#pragma unroll
+    for (int i = 0; i < KMAX; ++i) best.r[i] = a[i];
+    best.merge(c);
 }
 
-// Routes rows set*64 + lane of (b, h) on NW wavefronts. The waves split the
-// candidate blocks (wave w scores j = w, w + NW, ...), so the block index is uniform
-// across a wavefront: every 16-lane row loads the block's prototype with one
-// coalesced load (lane i of the row holds elements E*i .. E*i+E-1, E = DF/16),
-// one block ahead of its use, and the fma chain takes element d from lane d/E
-// of the row through a DPP row broadcast. Each lane keeps its row's KMAX best
-// route keys; wave m merges the waves' lists through `lists` (LDS,
-// [NW][KMAX][64] doubles) and returns true with the row's picks
-// (slots i >= ke: -1; slots no candidate filled: block i, the masked blocks
-// in ascending order); the other waves return false. With scores non-null,
-// every score of the row (-inf where masked) is written to scores[row * NB].
-// Called by every wavefront of the workgroup (two barriers inside).
-template <int FDT, int DF, int KMAX, int NW = kRouteWaves>
-__device__ __forceinline__ bool route_set(const void* __restrict__ f, int64_t fsb, int64_t fst, int64_t fsh,
-                                          const float* __restrict__ protos, int b, int h, int H, int64_t set,
-                                          int64_t Tq, int64_t NB, int bs, int ke, int causal, int64_t score_pos0,
-                                          float scale, float* __restrict__ scores, int m, double* lists,
-                                          int32_t (&picks)[KMAX]) {
+// Four consecutive forecast elements as fp32 (vec: 4-element aligned rows)
+template <int FDT>
+__device__ __forceinline__ float4 load_forecast4(const void* __restrict__ f, int64_t i, bool vec) {
+    if (vec) {
+        float o[4];
+        load_vec<FDT, 4>(f, i, o);
+        return make_float4(o[0], o[1], o[2], o[3]);
+    }
+    return make_float4(load_elem<FDT>(f, i), load_elem<FDT>(f, i + 1), load_elem<FDT>(f, i + 2),
+                       load_elem<FDT>(f, i + 3));
+}
+
+// Shape of a routing workgroup: NW wavefronts, of which PG x BG form scores:
+// row part p = w % PG takes RT tiles of 16 rows, block group w / PG every BG-th
+// tile of 16 blocks of a chunk (all of a chunk's CB = 16 TB BG blocks are
+// staged in LDS by the whole workgroup, the next chunk in flight).
+template <int DF, int NW, int PG, int BG, int RT, int TB>
+struct RouteShape {
+    static_assert(PG * BG <= NW, "score waves");
+    static constexpr int kRows = 16 * RT * PG;
+    static constexpr int kCB = 16 * TB * BG;
+    static constexpr int kRow = DF + 4;             // LDS row, floats: the 16 rows x 4 dims of an operand in 64 banks
+    static constexpr int kThreads = NW * kWave;
+    static constexpr int kFloats = kRows * kRow > 2 * kCB * kRow ? kRows * kRow : 2 * kCB * kRow;
+};
+
+// Routes rows row0 + r (r < nrows <= kRows) of (b, h). Scores are
+// v_mfma_f32_16x16x4_f32 products, 16 blocks (A, from LDS) x 16 rows (B, in
+// registers), the contraction walked in order: the instruction adds its four
+// terms as a sequential fma chain, so a score is the canonical chain
+// fma(f[d], p[d], acc), d ascending, bit for bit (checked for normal,
+// denormal, cancelling and infinite values; only the payload of a NaN may
+// differ, and a NaN score is formed again on the VALU). The matrix cores leave
+// the VALU to the top-k: lane l of the result holds blocks 4 (l / 16) .. +3 of row
+// l % 16, keeps that row's KMAX best route keys of its blocks, and the four
+// lanes of a row merge their lists at the end. On return best[rt] of a score
+// wavefront holds the list of row 16 (RT p + rt) + l % 16 over its block
+// group's blocks (merged further by the caller where BG > 1). With scores
+// non-null every score of the row (-inf where masked) is written to
+// scores[row * NB]. Called by every wavefront of the workgroup (barriers
+// inside; `lds` holds Shape::kFloats floats and is free again after the
+// caller's next barrier).
+template <int FDT, int DF, int KMAX, int NW, int PG, int BG, int RT, int TB>
+__device__ __forceinline__ void route_tiles(const void* __restrict__ f, int64_t fsb, int64_t fst, int64_t fsh,
+                                            const float* __restrict__ protos, int b, int h, int H, int64_t row0,
+                                            int nrows, int64_t Tq, int64_t NB, int bs, int causal,
+                                            int64_t score_pos0, float scale, float* __restrict__ scores,
+                                            float* lds, KeyTopK<KMAX> (&best)[RT]) {
 #pragma clang fp contract(off)
-    const int lane = threadIdx.x % kWave;
-    // the wave within its group of NW (a workgroup may route several sets at once)
-    const int w = __builtin_amdgcn_readfirstlane(static_cast<int>((threadIdx.x / kWave) % NW));
+    using Shape = RouteShape<DF, NW, PG, BG, RT, TB>;
+    constexpr int kRow = Shape::kRow;
+    constexpr int kS = DF / 4;                      // products per score tile; 16-byte chunks per row
+    const int tid = threadIdx.x;
+    const int lane = tid % kWave;
+    const int col16 = lane % 16;
+    const int grp = lane / 16;
+    const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int p = w % PG, bg = w / PG;
+    const bool scorer = bg < BG;                    // wave-uniform
     const float* __restrict__ pbh = protos + (static_cast<int64_t>(b) * NB * H + h) * DF;
     const int64_t pstride = static_cast<int64_t>(H) * DF;
-    const int64_t t = set * kWave + lane;
-    const bool active = t < Tq;
-    const int64_t tc = active ? t : Tq - 1;
-    const int64_t t_last = (set * kWave + kWave < Tq ? set * kWave + kWave : Tq) - 1;
-    int64_t limit = causal ? (score_pos0 + tc) / bs : NB - 1;
-    if (limit > NB - 1) limit = NB - 1;
+    const int64_t t_last = (row0 + nrows < Tq ? row0 + nrows : Tq) - 1;
     int64_t jmax64 = causal ? (score_pos0 + t_last) / bs : NB - 1;
     if (jmax64 > NB - 1) jmax64 = NB - 1;
-    // uniform: the block loop and the prototype addresses stay on the scalar unit
     const int jmax = __builtin_amdgcn_readfirstlane(static_cast<int>(jmax64));
 
-    float fr[DF];
-    {
-        constexpr int64_t V = FDT == SPARDA_F32 ? 4 : 8;  // elements per 16 bytes
-        const bool vec = (reinterpret_cast<uintptr_t>(f) & 15u) == 0 && fsb % V == 0 && fst % V == 0 && fsh % V == 0;
-        load_forecast_row<FDT, DF>(f, b * fsb + tc * fst + h * fsh, vec, fr);
-    }
-    const int64_t row = (static_cast<int64_t>(b) * H + h) * Tq + t;
-    float* srow = (scores != nullptr && active) ? scores + row * NB : nullptr;
-
-    KeyTopK<KMAX> best;
-    best.init();
-    constexpr int E = DF / 16;
-    constexpr int C = 2;  // blocks scored side by side
-    const int loff = (lane % 16) * E;  // this lane's elements of a prototype row
-    // prototype row of block min(jc, jmax) (a wave-uniform address), this lane's E elements
-    auto load_proto = [&](int jc, float (&o)[E]) __attribute__((always_inline)) {
-        const float* __restrict__ pb = pbh + static_cast<int64_t>(jc < jmax ? jc : jmax) * pstride;
-        load_f32<E>(pb + loff, o);
-    };
-    // scores blocks j, j + NW, ... (C of them, prototypes in pc) and
-    // pushes their keys
-    auto score = [&](int j, const float (&pc)[E][C]) __attribute__((always_inline)) {
-        float acc[C];
+    // chunk staging: thread -> 16-byte chunks e = tid + i kThreads of the chunk's rows (clamped to block jmax)
+    constexpr int kChunks = Shape::kCB * kS;
+    constexpr int kPer = (kChunks + Shape::kThreads - 1) / Shape::kThreads;
+    typedef float StageV __attribute__((ext_vector_type(4 * kPer)));
+    StageV pr;
+    auto fetch = [&](int c0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int c = 0; c < C; ++c) acc[c] = 0.0f;
-        row_fma_chains<E, DF, C>(fr, pc, acc);
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const int jc = j + c * NW;
-            const float sc = acc[c] * scale;
-            const bool ok = jc <= limit;  // limit <= jmax
-            if (srow && ok) srow[jc] = sc;
-            best.push(ok ? route_key(sc, static_cast<int32_t>(jc)) : 0.0);
+        for (int i = 0; i < kPer; ++i) {
+            const int e = tid + i * Shape::kThreads;
+            const int j = c0 + (e < kChunks ? e : 0) / kS;
+            const float4 x = *reinterpret_cast<const float4*>(pbh + (j < jmax ? j : jmax) * pstride + 4 * (e % kS));
+            pr[4 * i] = x.x; pr[4 * i + 1] = x.y; pr[4 * i + 2] = x.z; pr[4 * i + 3] = x.w;
         }
     };
-    // two prototype buffers used in turn, each loaded one step ahead of its use
-    constexpr int kStep = C * NW;
-    float pa[E][C], pz[E][C];
-    float tmp[E];
+    auto stash = [&](float* dst) __attribute__((always_inline)) {
 #pragma unroll
-    for (int c = 0; c < C; ++c) {
-        load_proto(w + c * NW, tmp);
-#pragma unroll
-        for (int e = 0; e < E; ++e) pa[e][c] = tmp[e];
-    }
-    for (int j = w; j <= jmax; j += 2 * kStep) {
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            load_proto(j + kStep + c * NW, tmp);
-#pragma unroll
-            for (int e = 0; e < E; ++e) pz[e][c] = tmp[e];
+        for (int i = 0; i < kPer; ++i) {
+            const int e = tid + i * Shape::kThreads;
+            if (kChunks % Shape::kThreads == 0 || e < kChunks)
+                *reinterpret_cast<float4*>(dst + (e / kS) * kRow + 4 * (e % kS)) =
+                    make_float4(pr[4 * i], pr[4 * i + 1], pr[4 * i + 2], pr[4 * i + 3]);
         }
-        score(j, pa);
-        if (j + kStep > jmax) break;  // uniform
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            load_proto(j + 2 * kStep + c * NW, tmp);
-#pragma unroll
-            for (int e = 0; e < E; ++e) pa[e][c] = tmp[e];
-        }
-        score(j + kStep, pz);
-    }
-    if (srow) {
-        for (int64_t j = w; j < NB; j += NW)
-            if (j > limit) srow[j] = -__builtin_inff();
-    }
+    };
 
-    // merge the waves' lists in the merging wave
-    __syncthreads();  // the previous set's merger has read its lists
-    if (w != m) {
-#pragma unroll
-        for (int i = 0; i < KMAX; ++i) lists[(w * KMAX + i) * kWave + lane] = best.r[i];
+    // the forecast rows through LDS into the B operands (step s: element 4 s + grp of row col16)
+    const int64_t V = 4;
+    const bool vec = (reinterpret_cast<uintptr_t>(f) & (FDT == SPARDA_F32 ? 15u : 7u)) == 0 && fsb % V == 0 &&
+                     fst % V == 0 && fsh % V == 0;
+    const int64_t fbase = b * fsb + h * fsh;
+    for (int e = tid; e < Shape::kRows * kS; e += Shape::kThreads) {
+        int64_t t = row0 + e / kS;
+        t = t < t_last ? t : t_last;
+        *reinterpret_cast<float4*>(lds + (e / kS) * kRow + 4 * (e % kS)) =
+            load_forecast4<FDT>(f, fbase + t * fst + 4 * (e % kS), vec);
     }
+    fetch(0);
     __syncthreads();
-    if (w != m) return false;
-    for (int o = 0; o < NW; ++o) {
-        if (o == m) continue;
-        double other[KMAX];
+    float fr[RT][kS];
+    int limit[RT];
+    float* srow[RT];
 #pragma unroll
-        for (int i = 0; i < KMAX; ++i) other[i] = lists[(o * KMAX + i) * kWave + lane];
-        best.merge(other);
+    for (int rt = 0; rt < RT; ++rt) {
+        const int r = 16 * (RT * p + rt) + col16;
+#pragma unroll
+        for (int s = 0; s < kS; ++s) fr[rt][s] = lds[r * kRow + 4 * s + grp];
+        const int64_t t = row0 + r < t_last ? row0 + r : t_last;
+        const int64_t lim = causal ? (score_pos0 + t) / bs : NB - 1;
+        limit[rt] = static_cast<int>(lim < jmax ? lim : jmax);
+        srow[rt] = (scores != nullptr && scorer && row0 + r <= t_last)
+                       ? scores + ((static_cast<int64_t>(b) * H + h) * Tq + row0 + r) * NB
+                       : nullptr;
+        best[rt].init();
     }
-    // slots not filled by a candidate take the masked blocks in ascending order
+    __syncthreads();  // the forecast's bytes are free
+
+    int cb = 0;
+    for (int c0 = 0; c0 <= jmax; c0 += Shape::kCB) {  // workgroup-uniform
+        float* buf = lds + cb * Shape::kCB * kRow;
+        stash(buf);
+        __syncthreads();
+        if (c0 + Shape::kCB <= jmax) fetch(c0 + Shape::kCB);
+        const int j0 = c0 + 16 * TB * bg;             // this wavefront's blocks of the chunk
+        if (scorer && j0 <= jmax) {
+            f32x4 acc[TB][RT];
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) acc[tb][rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const float* pa = buf + (16 * TB * bg + col16) * kRow + grp;
+#pragma unroll
+            for (int s = 0; s < kS; ++s)
+#pragma unroll
+                for (int tb = 0; tb < TB; ++tb) {
+                    const float a = pa[16 * tb * kRow + 4 * s];
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt)
+                        acc[tb][rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, fr[rt][s], acc[tb][rt], 0, 0, 0);
+                }
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    f32x4 v = acc[tb][rt];
+                    if (__ballot(__builtin_isunordered(v[0], v[1]) || __builtin_isunordered(v[2], v[3])) != 0ull) {
+                        // a NaN: the chain itself, for its payload
+                        const int64_t t = row0 + 16 * (RT * p + rt) + col16;
+                        const int64_t fi = fbase + (t < t_last ? t : t_last) * fst;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int j = j0 + 16 * tb + 4 * grp + i;
+                            if (j > limit[rt] || v[i] == v[i]) continue;
+                            float x = 0.0f;
+                            for (int d = 0; d < DF; ++d)
+                                x = __builtin_fmaf(pbh[j * pstride + d], load_elem<FDT>(f, fi + d), x);
+                            v[i] = x;
+                        }
+                    }
+                    double key[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int j = j0 + 16 * tb + 4 * grp + i;
+                        const bool ok = j <= limit[rt];
+                        const float sc = v[i] * scale;
+                        if (srow[rt] != nullptr && ok) srow[rt][j] = sc;
+                        key[i] = ok ? route_key(sc, j) : 0.0;
+                    }
+                    if (c0 == 0 && tb == 0) best[rt].init4(key);
+                    else best[rt].push4(key);
+                }
+        }
+        cb ^= 1;
+    }
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        if (srow[rt] != nullptr && bg == 0)
+            for (int64_t j = limit[rt] + 1 + grp; j < NB; j += 4) srow[rt][j] = -__builtin_inff();
+        if (scorer && 16 * TB * bg <= jmax) {  // wave-uniform: the others' lists are empty
+            merge_rows<16>(best[rt]);
+            merge_rows<32>(best[rt]);
+        }
+    }
+}
+
+// the row's picks (slots i >= ke: -1; slots no candidate filled: block i, the
+// masked blocks in ascending order)
+template <int KMAX>
+__device__ __forceinline__ void route_picks(const KeyTopK<KMAX>& best, int ke, int32_t (&picks)[KMAX]) {
 #pragma unroll
     for (int i = 0; i < KMAX; ++i) picks[i] = (i < ke) ? (best.r[i] == 0.0 ? i : route_key_index(best.r[i])) : -1;
-    return true;
 }
 
 }  // namespace sparda

@@ -81,19 +81,41 @@ struct KeyTopK {
 #pragma unroll
         for (int i = 0; i < KMAX; ++i) r[i] = 0.0;
     }
-    __device__ __forceinline__ void push(double x) {
+    // r <- the KMAX largest of r and four more keys
+    __device__ __forceinline__ void push4(double (&o)[4]) {
+        static_assert(KMAX >= 4 && (KMAX & (KMAX - 1)) == 0, "KMAX must be a power of two");
+        sort4(o);
 #pragma unroll
-        for (int i = 0; i < KMAX; ++i) {
-            const double lo = key_min(r[i], x);
-            asm("v_max_f64 %0, %0, %1" : "+v"(r[i]) : "v"(x));
-            x = lo;
-        }
+        for (int i = 0; i < 4; ++i) r[KMAX - 1 - i] = key_max(r[KMAX - 1 - i], o[i]);
+        clean();
+    }
+    // an empty list <- four keys
+    __device__ __forceinline__ void init4(double (&o)[4]) {
+        sort4(o);
+#pragma unroll
+        for (int i = 0; i < KMAX; ++i) r[i] = i < 4 ? o[i < 4 ? i : 0] : 0.0;
+    }
+    static __device__ __forceinline__ void order(double& a, double& b) {  // a >= b
+        const double hi = key_max(a, b);
+        b = key_min(a, b);
+        a = hi;
+    }
+    static __device__ __forceinline__ void sort4(double (&o)[4]) {
+        order(o[0], o[1]);
+        order(o[2], o[3]);
+        order(o[0], o[2]);
+        order(o[1], o[3]);
+        order(o[1], o[2]);
     }
     // r <- the KMAX largest of r and o (both descending): bitonic merge
     __device__ __forceinline__ void merge(const double (&o)[KMAX]) {
         static_assert((KMAX & (KMAX - 1)) == 0, "KMAX must be a power of two");
 #pragma unroll
         for (int i = 0; i < KMAX; ++i) r[i] = key_max(r[i], o[KMAX - 1 - i]);
+        clean();
+    }
+    // a bitonic list into descending order
+    __device__ __forceinline__ void clean() {
 #pragma unroll
         for (int s = KMAX / 2; s > 0; s >>= 1) {
 #pragma unroll
