@@ -763,10 +763,22 @@ static bool compact_layout_ok(int64_t R, int64_t q_sb, int64_t q_st, int64_t q_s
     return true;
 }
 
-// 128-token windows wherever their LDS fits (R <= 3): twice the tokens of a
-// 64-token window fill the tiles of each selected block. The output is the same
-// bit for bit: a column's sums do not depend on its tile mates.
-static int pick_window(int64_t R, int64_t, int64_t) { return R <= 3 ? 128 : 64; }
+// The query window of a call: the narrowest whose workgroups (one per CU at a
+// time) still start together, up to a quarter past one per CU; 128 tokens where
+// even those take several rounds, the tiles of a wider window being fuller (64
+// for R = 4, whose accumulators for 128 tokens do not fit the LDS). A
+// workgroup's time is about 20 us of routing, set-up and load latency
+// plus 0.35 us a token (12/4 heads, 64-key blocks, T=4096). Measured at B=1, 12/4
+// heads, top-8 of 64-key blocks, us at 128 / 64 / 32 / 16 tokens: T=1024 56 / 40 /
+// 35 / 30, T=2048 63 / 53 / 43 / 53, T=3000 71 / 59 / 65 / 80, T=4096 83 / 60 / 76,
+// T=5003 85 / 78 / 103, T=8192 92 / 113; B=4, T=4096 129 / 181. The output is the
+// same bit for bit: a column's sums do not depend on its tile mates.
+static int pick_window(int64_t R, int64_t BH, int64_t T) {
+    const int widest = R <= 3 ? 128 : 64;
+    for (int W = 16; W < widest; W *= 2)
+        if (4 * BH * cdiv(T, W) <= 5 * kCCus) return W;
+    return widest;
+}
 
 // Polls an ordering wait makes before the workgroup abandons it (the window
 // is then NaN and the status word flags it). SPARDA_PREFILL_WAIT_LIMIT
