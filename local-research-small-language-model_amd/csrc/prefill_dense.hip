@@ -2,15 +2,22 @@
 // the reference's dense fallback (model/attention/sparse.py:201-224: layer 0,
 // no forecast, or at most two KV blocks) without selection lists.
 //
-// One workgroup of 8 wavefronts serves one (sequence b, KV head g, window of
-// 128 query tokens); wavefront w owns tokens [16w, 16w+16) of the window for
-// all R = Hq/Hkv query heads of the group: 16R columns (column c -> token
-// 16w + c / R, head c % R), R tiles of 16 columns whose Q operands stay in
-// registers. The workgroup walks the KV blocks of 64 keys in ascending order
-// up to its last token's block; each block's K and V are staged once in LDS
-// (double-buffered; the next block is loaded into registers while the
-// current one is computed) and shared by all 128 tokens and R heads. Per tile
-// and block, with v_mfma_f32_16x16x32_bf16:
+// One workgroup of CW x KG = 8 wavefronts serves one (sequence b, KV head g,
+// window of 16 CW query tokens): CW token waves, each with the tokens
+// [16w, 16w+16) of the window for all R = Hq/Hkv query heads of the group: 16R
+// columns (column c -> token c / R, head c % R), R tiles of 16 columns whose Q
+// operands stay in registers; and KG key groups of CW waves, of which group kg
+// walks the KV blocks kg, kg + KG, ... of 64 keys in ascending order up to the
+// window's last token's block. Each block's K and V are staged once in LDS by
+// their group (double-buffered; the next block is loaded into registers while
+// the current one is computed) and shared by the window's tokens and R heads.
+// The groups share the columns' references, so their O and row sums are added
+// at the end, in group order. Small windows times key groups keep the number of
+// workgroups well past one per CU, so that the causal triangle balances: at B=1,
+// T=8192, 12/4 heads 128 us (800 TFLOP/s) against 231 with one group and 128-token
+// windows (256 workgroups, the heaviest twice the mean). Bound by issue: a wave's
+// exponentials and products take turns, so that the matrix cores are busy about
+// 40% of the time. Per tile and block, with v_mfma_f32_16x16x32_bf16:
 //     S^T[key, col] = K[key, :] . Q[col, :]           (8 MFMA)
 //     P = exp2(S * scale log2 e - ref[col]), bf16      (fp32 exponent)
 //     O^T[d, col]  += V^T[d, key] . P^T[key, col]      (8 MFMA)
@@ -45,17 +52,37 @@ namespace {
 
 constexpr int kDBs = 64;                 // keys per KV block
 constexpr int kDD = 64;                  // head dim
-constexpr int kDWaves = 8;               // wavefronts per workgroup (dense)
-constexpr int kLWaves = 4;               // wavefronts per workgroup (listed: one 64-token query block)
+constexpr int64_t kDCus = 256;           // compute units: one dense workgroup each
+constexpr int kLTok = 4;                 // token waves of a listed workgroup (one 64-token query block)
 constexpr int kDKRow = kDD + 8;          // K row in LDS, bf16 elements (144 B)
 constexpr int kDVRow = kDD + 16;         // V row in LDS, bf16 elements (160 B)
 constexpr float kDLog2e = 1.4426950408889634f;
 constexpr float kDGuard = 18446744073709551616.0f;  // 2^64: a row sum past it means a score far above ref
 
+template <int KG>
+struct DenseStage {
+    uint16_t k[2][KG][kDBs * kDKRow];
+    uint16_t v[2][KG][kDBs * kDVRow];
+};
+
+// partial O and row sums of the KG - 1 later key groups, added into the first
+// group's after the walk (lane-linear: every access is one row of 64 lanes)
+template <int R, int CW, int KG>
+struct DenseMerge {
+    f32x4 o[KG - 1][CW][R * 4][kWave];
+    float l[KG - 1][CW][R][16];
+};
+template <int R, int CW>
+struct DenseMerge<R, CW, 1> {};
+
+template <int R, int CW, int KG>
 struct DenseSmem {
-    uint16_t k[2][kDBs * kDKRow];
-    uint16_t v[2][kDBs * kDVRow];
+    union {
+        DenseStage<KG> st;
+        DenseMerge<R, CW, KG> mg;
+    };
     int flag;                             // some column's row sum passed kDGuard
+    int arrived[KG];                      // waves of a key group past its barriers
 };
 
 // the chunked lists' inputs and outputs (LISTED only)
@@ -69,21 +96,24 @@ struct ChunkArgs {
 
 }  // namespace
 
-template <int R, bool LISTED>
-__global__ void __launch_bounds__((LISTED ? kLWaves : kDWaves) * kWave, 2)
+template <int R, bool LISTED, int CW, int KG>
+__global__ void __launch_bounds__(CW * KG * kWave, 2)
 prefill_dense_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, int64_t q_sh,
                      const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, int64_t kv_sb, int64_t kv_st,
                      int64_t kv_sh, int64_t T, int H, int64_t NBq, int causal, float scale_log2,
                      uint16_t* __restrict__ out, int64_t out_sb, int64_t out_st, ChunkArgs ch) {
-    constexpr int kNW = LISTED ? kLWaves : kDWaves;
-    constexpr int kThreads = kNW * kWave;
-    constexpr int kWin = 16 * kNW;               // query tokens per workgroup
+    constexpr int kThreads = CW * kWave;         // threads of a key group: they stage its block
+    constexpr int kWin = 16 * CW;                // query tokens per workgroup
     constexpr int kSR = kDBs * 8 / kThreads;     // 16-byte K (and V) chunks each thread stages per block
-    __shared__ DenseSmem sm;
+    static_assert(!LISTED || (CW == kLTok && KG == 1), "a listed workgroup is one 64-token query block");
+    __shared__ DenseSmem<R, CW, KG> sm;
     __shared__ ChunkLds cl;
-    const int tid = threadIdx.x;
-    const int lane = tid % kWave;
-    const int wave = tid / kWave;
+    const int lane = threadIdx.x % kWave;
+    // wave-uniform (scalar registers): the token wave, and the key group, which
+    // walks the blocks kg, kg + KG, ...
+    const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+    const int wave = wv % CW, kg = wv / CW;
+    const int tid = wave * kWave + lane;         // thread within its key group
     const int col16 = lane % 16;
     const int grp = lane / 16;
 
@@ -130,7 +160,8 @@ prefill_dense_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st,
     clear();
 #pragma unroll
     for (int tt = 0; tt < R; ++tt) ref[tt] = -__builtin_inff();
-    if (tid == 0) sm.flag = 0;  // ordered before its uses by the staging barrier
+    if (threadIdx.x < KG) sm.arrived[threadIdx.x] = 0;
+    if (threadIdx.x == 0) sm.flag = 0;  // ordered before its uses by the staging barrier
 
     // staging: thread -> 16-byte chunks (rows tid / 8 + i * kThreads / 8, column
     // tid % 8) of K and of V; rows past T (a ragged last block) read row T-1
@@ -143,12 +174,16 @@ prefill_dense_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st,
     // uint4 handed between the lambdas would be placed in scratch memory)
     typedef unsigned int StageV __attribute__((ext_vector_type(4 * kSR)));
     auto fetch = [&](int j, StageV& kv_k, StageV& kv_v) __attribute__((always_inline)) {
+        const int64_t row0 = static_cast<int64_t>(j) * kDBs;  // uniform: the block's base is scalar
+        const int last = static_cast<int>(T - 1 - row0 < kDBs - 1 ? T - 1 - row0 : kDBs - 1);
+        const uint16_t* kb = kbase + row0 * kv_st;
+        const uint16_t* vb = vbase + row0 * kv_st;
 #pragma unroll
         for (int i = 0; i < kSR; ++i) {
-            int64_t s = static_cast<int64_t>(j) * kDBs + srow + i * kRowStep;
-            s = s < T ? s : T - 1;
-            const uint4 a = *reinterpret_cast<const uint4*>(kbase + s * kv_st + scol);
-            const uint4 c = *reinterpret_cast<const uint4*>(vbase + s * kv_st + scol);
+            int r = srow + i * kRowStep;
+            r = r < last ? r : last;
+            const uint4 a = *reinterpret_cast<const uint4*>(kb + (r * kv_st + scol));
+            const uint4 c = *reinterpret_cast<const uint4*>(vb + (r * kv_st + scol));
             kv_k[4 * i] = a.x; kv_k[4 * i + 1] = a.y; kv_k[4 * i + 2] = a.z; kv_k[4 * i + 3] = a.w;
             kv_v[4 * i] = c.x; kv_v[4 * i + 1] = c.y; kv_v[4 * i + 2] = c.z; kv_v[4 * i + 3] = c.w;
         }
@@ -156,9 +191,9 @@ prefill_dense_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st,
     auto stash = [&](int buf, const StageV& kv_k, const StageV& kv_v) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < kSR; ++i) {
-            *reinterpret_cast<uint4*>(&sm.k[buf][(srow + i * kRowStep) * kDKRow + scol]) =
+            *reinterpret_cast<uint4*>(&sm.st.k[buf][kg][(srow + i * kRowStep) * kDKRow + scol]) =
                 uint4{kv_k[4 * i], kv_k[4 * i + 1], kv_k[4 * i + 2], kv_k[4 * i + 3]};
-            *reinterpret_cast<uint4*>(&sm.v[buf][(srow + i * kRowStep) * kDVRow + scol]) =
+            *reinterpret_cast<uint4*>(&sm.st.v[buf][kg][(srow + i * kRowStep) * kDVRow + scol]) =
                 uint4{kv_v[4 * i], kv_v[4 * i + 1], kv_v[4 * i + 2], kv_v[4 * i + 3]};
         }
     };
@@ -183,12 +218,45 @@ prefill_dense_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st,
     }
     // the u-th block walked
     auto blk = [&](int u) __attribute__((always_inline)) -> int {
-        if constexpr (LISTED) return cl.lst[u];
+        if constexpr (LISTED) return __builtin_amdgcn_readfirstlane(static_cast<int>(cl.lst[u]));
         else return u;
     };
 
-    // mode 0: P against the references (the first block walked sets them
-    // unless `keep`); mode 1: scores only, the exact column maxima into ref
+    // the columns' scores against the first block walked, which every key group
+    // takes its references from (one group's slot, read by all)
+    auto set_refs = [&](int j) __attribute__((always_inline)) {
+        bf16x8 ka[4][2];
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk)
+                ka[n][kk] = lds_read8(&sm.st.k[0][0][(16 * n + col16) * kDKRow + 32 * kk + 8 * grp]);
+        const int64_t key0 = static_cast<int64_t>(j) * kDBs;
+        const bool edge = causal ? key0 + kDBs - 1 > w_first : key0 + kDBs > T;
+#pragma unroll
+        for (int tt = 0; tt < R; ++tt) {
+            f32x4 s[4];
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+                s[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[n][0], qreg[tt][0], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                s[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[n][1], qreg[tt][1], s[n], 0, 0, 0);
+            }
+            if (edge) {
+                const int64_t lim64 = causal ? t0 + tok[tt] - key0 : T - 1 - key0;
+                const int lim = static_cast<int>(lim64 < kDBs ? lim64 : kDBs);
+#pragma unroll
+                for (int n = 0; n < 4; ++n)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (16 * n + 4 * grp + i > lim) s[n][i] = -__builtin_inff();
+            }
+            ref[tt] = pair32_max(pair16_max(max_acc(s, -__builtin_inff()))) * scale_log2;  // block's column max, log2 units
+        }
+    };
+
+    // mode 0: P against the references (with one key group the first block
+    // walked sets them unless `keep`); mode 1: scores only, the exact column
+    // maxima of the group's blocks into ref
     auto compute = [&](int buf, int j, bool first, int mode, bool keep) __attribute__((always_inline)) {
         // K A operands: key 16n + col16, dims 32kk + 8grp .. +7
         bf16x8 ka[4][2];
@@ -196,7 +264,7 @@ prefill_dense_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st,
         for (int n = 0; n < 4; ++n)
 #pragma unroll
             for (int kk = 0; kk < 2; ++kk)
-                ka[n][kk] = lds_read8(&sm.k[buf][(16 * n + col16) * kDKRow + 32 * kk + 8 * grp]);
+                ka[n][kk] = lds_read8(&sm.st.k[buf][kg][(16 * n + col16) * kDKRow + 32 * kk + 8 * grp]);
         // V^T A operands, read transposed from the row-major tile
         bf16x8 va[4][2];
         if (mode == 0) {
@@ -206,7 +274,7 @@ prefill_dense_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st,
             for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
                 for (int m = 0; m < 2; ++m) {
-                    const uint16_t* base = &sm.v[buf][(32 * m + rsub) * kDVRow + 16 * dt + csub];
+                    const uint16_t* base = &sm.st.v[buf][kg][(32 * m + rsub) * kDVRow + 16 * dt + csub];
                     const i16x4 lo = lds_read_tr(base);
                     const i16x4 hi = lds_read_tr(base + 16 * kDVRow);
                     va[dt][m] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -232,8 +300,8 @@ prefill_dense_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st,
                     for (int i = 0; i < 4; ++i)
                         if (16 * n + 4 * grp + i > lim) s[n][i] = -__builtin_inff();
             }
-            if (mode == 1 || (first && !keep)) {  // wave-uniform
-                const float cand = pair32_max(pair16_max(max16_nn(s))) * scale_log2;  // block's column max, log2 units
+            if (mode == 1 || (KG == 1 && first && !keep)) {  // wave-uniform
+                const float cand = pair32_max(pair16_max(max_acc(s, -__builtin_inff()))) * scale_log2;  // block's column max, log2 units
                 ref[tt] = mode == 1 ? fmaxf(ref[tt], cand) : cand;
                 if (mode == 1) continue;
             }
@@ -263,24 +331,51 @@ prefill_dense_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st,
         }
     };
 
-    // block u is computed from buffer u & 1 while block u + 1 is in registers;
-    // one barrier per block orders its stash before the reads of the next
-    // (nk, nv: block blk(0) already loaded when have0)
+    // step i: group kg computes block i KG + kg from buffer i & 1 while its
+    // block of the next step is in registers; one barrier per step orders its
+    // stash before the reads of the next (nk, nv: block blk(0) already loaded
+    // when have0, one key group only)
+    // The barrier of a step joins the waves of one key group only: the groups share
+    // nothing until the merge, and out of step one group's exponentials run
+    // beside the other's products (in step, every wave of a SIMD wants the same
+    // unit: 4 to 12% slower). A wave arrives once its LDS accesses of the step are done; all waves of
+    // the workgroup are resident, so every one arrives.
+    int phase = 0;
+    auto group_sync = [&]() __attribute__((always_inline)) {
+        if constexpr (KG == 1) {
+            __syncthreads();
+        } else {
+            phase += CW;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            if (lane == 0) __hip_atomic_fetch_add(&sm.arrived[kg], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            while (__builtin_amdgcn_readfirstlane(__hip_atomic_load(&sm.arrived[kg], __ATOMIC_RELAXED,
+                                                                    __HIP_MEMORY_SCOPE_WORKGROUP)) < phase)
+                __builtin_amdgcn_s_sleep(1);
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        }
+    };
+    const int steps = (nblk + KG - 1) / KG;  // workgroup-uniform
     auto walk = [&](int mode, bool keep, StageV nk, StageV nv, bool have0) __attribute__((always_inline)) {
-        if (!have0) fetch(blk(0), nk, nv);
-        stash(0, nk, nv);
-        if (nblk > 1) fetch(blk(1), nk, nv);
+        if (!have0 && kg < nblk) fetch(blk(kg), nk, nv);
+        if (kg < nblk) stash(0, nk, nv);
+        if (kg + KG < nblk) fetch(blk(kg + KG), nk, nv);
         __syncthreads();
-        for (int u = 0; u < nblk; ++u) {
-            const int buf = u & 1;
+        if (KG > 1 && mode == 0 && !keep) {
+            if (w_live) set_refs(blk(0));
+            __syncthreads();  // the first block has been read by every group
+        }
+        for (int i = 0; i < steps; ++i) {
+            const int buf = i & 1;
+            const int u = i * KG + kg;
             // wave-uniform: blocks past this wavefront's tokens are skipped
             if (u < w_nblk) compute(buf, blk(u), u == 0, mode, keep);
-            if (u + 1 < nblk) {
+            if (u + KG < nblk) {
                 stash(buf ^ 1, nk, nv);
-                if (u + 2 < nblk) fetch(blk(u + 2), nk, nv);
+                if (u + 2 * KG < nblk) fetch(blk(u + 2 * KG), nk, nv);
             }
-            __syncthreads();
+            group_sync();
         }
+        if (KG > 1) __syncthreads();  // every group's last reads of the staging bytes
     };
     walk(0, false, nk0, nv0, LISTED);
     // a row sum past 2^64 (or not finite): a score more than 64 log2-units above
@@ -296,8 +391,41 @@ prefill_dense_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st,
 #pragma unroll
         for (int tt = 0; tt < R; ++tt) ref[tt] = -__builtin_inff();
         walk(1, true, nk0, nv0, false);  // the exact column maxima
+        if constexpr (KG > 1) {
+            // of every group's blocks (the walk's last barrier freed the staging bytes)
+#pragma unroll
+            for (int tt = 0; tt < R; ++tt)
+                if (grp == 0) reinterpret_cast<float*>(&sm.st)[((kg * CW + wave) * R + tt) * 16 + col16] = ref[tt];
+            __syncthreads();
+#pragma unroll
+            for (int tt = 0; tt < R; ++tt)
+                for (int o_ = 0; o_ < KG; ++o_)
+                    ref[tt] = fmaxf(ref[tt], reinterpret_cast<float*>(&sm.st)[((o_ * CW + wave) * R + tt) * 16 + col16]);
+            __syncthreads();
+        }
         clear();
         walk(0, true, nk0, nv0, false);  // against them: every P <= 1
+    }
+    if constexpr (KG > 1) {
+        // the groups' sums share their references: plain additions, in group order
+        if (kg > 0) {
+#pragma unroll
+            for (int tt = 0; tt < R; ++tt) {
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt) sm.mg.o[kg - 1][wave][4 * tt + dt][lane] = o[tt][dt];
+                if (lane < 16) sm.mg.l[kg - 1][wave][tt][lane] = ol[tt][0];
+            }
+        }
+        __syncthreads();
+        if (kg > 0) return;
+#pragma unroll
+        for (int o_ = 0; o_ < KG - 1; ++o_)
+#pragma unroll
+            for (int tt = 0; tt < R; ++tt) {
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt) o[tt][dt] += sm.mg.o[o_][wave][4 * tt + dt][lane];
+                ol[tt][0] += sm.mg.l[o_][wave][tt][col16];
+            }
     }
 
     // ---- epilogue: out[b, t, h*64 + d] = O / l ----
@@ -336,21 +464,28 @@ int launch_prefill_dense(const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh
                          int64_t kv_sb, int64_t kv_st, int64_t kv_sh, int64_t B, int64_t T, int64_t Hq,
                          int64_t Hkv, int causal, float scale, void* out, int64_t out_sb, int64_t out_st,
                          hipStream_t stream) {
-    const int64_t NBq = cdiv(T, 16 * kDWaves);
     const int64_t R = Hq / Hkv;
-    dim3 grid(static_cast<unsigned>(B * Hkv * NBq));
     const float sl = scale * kDLog2e;
-#define SPARDA_DN(R_)                                                                                      \
-    hipLaunchKernelGGL((prefill_dense_kernel<R_, false>), grid, dim3(kDWaves * kWave), 0, stream,          \
+#define SPARDA_DN(R_, CW_, KG_)                                                                            \
+    hipLaunchKernelGGL((prefill_dense_kernel<R_, false, CW_, KG_>),                                        \
+                       dim3(static_cast<unsigned>(B * Hkv * cdiv(T, 16 * CW_))), dim3(CW_ * KG_ * kWave), 0, stream, \
                        static_cast<const uint16_t*>(q), q_sb, q_st, q_sh, static_cast<const uint16_t*>(k), \
-                       static_cast<const uint16_t*>(v), kv_sb, kv_st, kv_sh, T, static_cast<int>(Hkv), NBq, \
-                       causal, sl, static_cast<uint16_t*>(out), out_sb, out_st, ChunkArgs{})
+                       static_cast<const uint16_t*>(v), kv_sb, kv_st, kv_sh, T, static_cast<int>(Hkv),     \
+                       cdiv(T, 16 * CW_), causal, sl, static_cast<uint16_t*>(out), out_sb, out_st, ChunkArgs{})
+#define SPARDA_DN_W(R_)                         \
+    if (wide) SPARDA_DN(R_, 4, 2);              \
+    else SPARDA_DN(R_, 2, 4);
+    // 64-token windows from 5/4 workgroups per CU on, else 32-token windows of
+    // four key groups (12/4 heads: 49 us against 64 at T=4096, 256 windows of 64;
+    // 99 us against 91 at T=6000, 376 windows; 25 against 36 at T=2048)
+    const bool wide = 4 * B * Hkv * cdiv(T, 64) > 5 * kDCus;
     switch (R) {
-        case 1: SPARDA_DN(1); break;
-        case 2: SPARDA_DN(2); break;
-        case 3: SPARDA_DN(3); break;
-        default: SPARDA_DN(4); break;
+        case 1: SPARDA_DN_W(1); break;
+        case 2: SPARDA_DN_W(2); break;
+        case 3: SPARDA_DN_W(3); break;
+        default: SPARDA_DN_W(4); break;
     }
+#undef SPARDA_DN_W
 #undef SPARDA_DN
     return check_hip(hipGetLastError(), "prefill_dense_kernel");
 }
@@ -374,7 +509,7 @@ int launch_prefill_chunked(const void* q, int64_t q_sb, int64_t q_st, int64_t q_
     const ChunkArgs ch{topk, static_cast<int>(ke), static_cast<int>(top_k), static_cast<int>(cut), sel, n_sel,
                        static_cast<int>(sel != nullptr ? cap : 0)};
 #define SPARDA_CH(R_)                                                                                      \
-    hipLaunchKernelGGL((prefill_dense_kernel<R_, true>), grid, dim3(kLWaves * kWave), 0, stream,           \
+    hipLaunchKernelGGL((prefill_dense_kernel<R_, true, kLTok, 1>), grid, dim3(kLTok * kWave), 0, stream,   \
                        static_cast<const uint16_t*>(q), q_sb, q_st, q_sh, static_cast<const uint16_t*>(k), \
                        static_cast<const uint16_t*>(v), kv_sb, kv_st, kv_sh, T, static_cast<int>(Hkv), NBq, \
                        1, sl, static_cast<uint16_t*>(out), out_sb, out_st, ch)
