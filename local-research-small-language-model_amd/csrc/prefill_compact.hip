@@ -178,7 +178,9 @@ prefill_compact_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_s
     static_assert(BS == 64 || BS == 32, "KV blocks of 64 or 32 keys");
     constexpr int kSub = BS / 16;  // 16-key sub-tiles of a block (the M side of S^T)
     constexpr int kHalf = BS / 32; // 32-key halves of a block (the K side of O^T)
-    // tiles per work item: three for 64-key blocks, two for 32-key blocks
+    // most tiles per work item: a block's tiles are shared evenly among as few
+    // items as that allows (four as 2 + 2: a lone tile pays a whole block's loads,
+    // 131 us against 126 at B=4, T=4096). Three for 64-key blocks, two for 32-key blocks
     // (whose items then hold fewer keys; three measured 6-7% slower there,
     // 1-13% faster for 64-key blocks)
     constexpr int kCChunk = BS == 64 ? 3 : 2;
@@ -322,6 +324,7 @@ prefill_compact_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_s
             const int nt = mask_count(M);
             const int tiles = (R * nt + 15) / 16;
             const int chunks = nz ? (tiles + kCChunk - 1) / kCChunk : 0;
+            const int per = nz ? (tiles + chunks - 1) / chunks : 0;
             const int rk = nz ? nt : 0;
             int sc = chunks, sr = rk;  // inclusive prefix sums over the lanes
 #pragma unroll
@@ -339,7 +342,7 @@ prefill_compact_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_s
                 sm.uofs[pos] = static_cast<uint16_t>(nrk + sr - rk);
                 jmap[j] = static_cast<uint16_t>(pos);
                 for (int cc = 0; cc < chunks; ++cc)
-                    sm.items[item0 + cc] = static_cast<uint32_t>(pos) | (static_cast<uint32_t>(cc * kCChunk) << 16);
+                    sm.items[item0 + cc] = static_cast<uint32_t>(pos) | (static_cast<uint32_t>(cc * per) << 16);
             }
             nu += __popcll(bal);
             ni += __shfl(sc, kWave - 1, kWave);
@@ -505,7 +508,8 @@ prefill_compact_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_s
         const int rofs = sm.uofs[u];
         const int ncol = R * (sm.uofs[u + 1] - rofs);
         const int tiles = (ncol + 15) / 16;
-        const int nt = (i0 + kCChunk < tiles ? i0 + kCChunk : tiles) - i0;  // 1 .. kCChunk
+        const int chunks = (tiles + kCChunk - 1) / kCChunk, per = (tiles + chunks - 1) / chunks;
+        const int nt = (i0 + per < tiles ? i0 + per : tiles) - i0;  // 1 .. kCChunk
         // causal: a block that ends past the window's first token holds keys
         // beyond some selecting tokens (key j*BS + i is allowed up to token t0 + tk)
         const bool diag = causal && (static_cast<int64_t>(j) + 1) * BS - 1 > t0;
@@ -771,7 +775,8 @@ static bool compact_layout_ok(int64_t R, int64_t q_sb, int64_t q_st, int64_t q_s
 // plus 0.35 us a token (12/4 heads, 64-key blocks, T=4096). Measured at B=1, 12/4
 // heads, top-8 of 64-key blocks, us at 128 / 64 / 32 / 16 tokens: T=1024 56 / 40 /
 // 35 / 30, T=2048 63 / 53 / 43 / 53, T=3000 71 / 59 / 65 / 80, T=4096 83 / 60 / 76,
-// T=5003 85 / 78 / 103, T=8192 92 / 113; B=4, T=4096 129 / 181. The output is the
+// T=5003 85 / 78 / 103, T=8192 92 / 113; B=4, T=4096 129 / 181 (before the items of a
+// block were evened out, which took 4% off the widest). The output is the
 // same bit for bit: a column's sums do not depend on its tile mates.
 static int pick_window(int64_t R, int64_t BH, int64_t T) {
     const int widest = R <= 3 ? 128 : 64;
