@@ -823,7 +823,7 @@ def bench_teacher(args, torch, sparda, synth):
         err = float((mass - ref[0].float()).abs().max())
         us_kernel = events_ms(lambda: sparda.teacher_block_mass(q, k, BS), 10, torch) * 1e3
         us_mat = events_ms(materialised, 3, torch) * 1e3
-    flop = 2 * (4.0 * D * PB * HQ * PT * (PT + 1) / 2)  # QK^T over the causal pairs, two passes
+    flop = 2.0 * D * PB * HQ * PT * (PT + 1) / 2  # QK^T over the causal pairs, one pass, 2 flop per multiply-add
     return {
         "workload": f"teacher block mass, B={PB} T={PT} Hq={HQ} Hkv={HKV} D={D} block={BS}, causal, bf16",
         "us_kernel": round(us_kernel, 1),
