@@ -24,8 +24,9 @@
 // x x^T, formed on the matrix cores from the staged x fragments (each of the
 // two wavefronts that share the rows takes every second row tile).
 // Bound by the latency of a step's loads and LDS reads (the matrix cores are busy
-// a third of the time): 62 us = 630 TFLOP/s at M = 16384, N = 1536, C = 768, from
-// 72 us with 128 x 128 tiles, the squares on the VALU and 2-byte stores.
+// 40% of the time): 60 us = 647 TFLOP/s at M = 16384, N = 1536, C = 768, from
+// 72 us with 128 x 128 tiles, the squares on the VALU and 2-byte stores (62 with
+// padded rows staged before the products; M = 8192 37.9 then, 35.2 now).
 #include "common.h"
 #include "kernels.h"
 #include "rows.h"
