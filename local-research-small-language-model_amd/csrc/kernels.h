@@ -226,7 +226,7 @@ int offload_append_at(sparda_offload_t h, const void* k, const void* v, int64_t 
 
 // fp32 on the matrix cores (D = 64, blocks of 64 or 32 keys); sel nullptr: dense
 bool prefill_f32_supported(int dtype, int64_t T, int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int64_t B,
-                           const int32_t* sel, int64_t q_sb, int64_t q_st, int64_t q_sh, int64_t kv_sb,
+                           const int32_t* sel, int64_t cap, int64_t q_sb, int64_t q_st, int64_t q_sh, int64_t kv_sb,
                            int64_t kv_st, int64_t kv_sh, int64_t out_sb, int64_t out_st, const void* q,
                            const void* k, const void* v, const void* out);
 int launch_prefill_f32(const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh, const void* k, const void* v,

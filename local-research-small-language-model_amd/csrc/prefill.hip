@@ -348,7 +348,7 @@ int launch_prefill(const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh, cons
                                out_st, q, k, v, out))
         return launch_prefill_mfma(q, q_sb, q_st, q_sh, k, v, kv_sb, kv_st, kv_sh, sel, n_sel, cap,
                                    B, T, Hq, Hkv, bs, causal, scale, out, out_sb, out_st, stream);
-    if (prefill_f32_supported(dtype, T, Hq, Hkv, D, bs, B, sel, q_sb, q_st, q_sh, kv_sb, kv_st, kv_sh, out_sb,
+    if (prefill_f32_supported(dtype, T, Hq, Hkv, D, bs, B, sel, cap, q_sb, q_st, q_sh, kv_sb, kv_st, kv_sh, out_sb,
                               out_st, q, k, v, out))
         return launch_prefill_f32(q, q_sb, q_st, q_sh, k, v, kv_sb, kv_st, kv_sh, sel, n_sel, cap, B, T, Hq, Hkv, bs,
                                   causal, scale, out, out_sb, out_st, stream);

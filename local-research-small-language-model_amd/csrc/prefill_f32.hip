@@ -40,7 +40,6 @@ namespace {
 constexpr int kFWaves = 4;
 constexpr int kFThreads = kFWaves * kWave;
 constexpr int kFMaxNB = 2048;                       // KV blocks a token mask array covers
-constexpr int kFMaxDup = 16 * kMaxSelCap;           // repeated list entries of a tile
 constexpr float kFLog2e = 1.4426950408889634f;
 
 struct F32Merge {
@@ -52,9 +51,8 @@ struct F32Smem {
         uint32_t mask[kFMaxNB];                     // tokens that listed block j (set-up)
         F32Merge mg;                                // the later wavefronts' partials (after the walk)
     };
-    uint32_t ent[kFMaxNB + kFMaxDup];               // block << 16 | token mask
-    uint32_t dup[kFMaxDup];
-    int n_ent, n_dup;
+    uint32_t ent[kFMaxNB];                          // block << 16 | token mask
+    int n_ent;
 };
 
 }  // namespace
@@ -107,19 +105,13 @@ prefill_f32_kernel(const float* __restrict__ q, int64_t q_sb, int64_t q_st, int6
     int n_ent = jmax + 1;
     if (sel != nullptr) {
         for (int i = tid; i <= jmax; i += kFThreads) sm.mask[i] = 0u;
-        if (tid == 0) sm.n_dup = 0;
         __syncthreads();
         const int64_t row0 = bg * T + t0;
         for (int e = tid; e < nt * cap; e += kFThreads) {
             const int tt = e / cap, i = e - tt * cap;
             const int j = sel[(row0 + tt) * cap + i];
             const int tlim = causal ? static_cast<int>((t0 + tt) / BS) : jmax;  // later blocks hold no allowed key
-            if (i < n_sel[row0 + tt] && j >= 0 && j <= tlim) {
-                const uint32_t bit = 1u << tt;
-                // a block listed twice counts twice: an entry of its own
-                if (atomicOr(&sm.mask[j], bit) & bit)
-                    sm.dup[atomicAdd(&sm.n_dup, 1)] = static_cast<uint32_t>(j) << 16 | bit;
-            }
+            if (i < n_sel[row0 + tt] && j >= 0 && j <= tlim) atomicOr(&sm.mask[j], 1u << tt);  // a repeat counts once
         }
         __syncthreads();
         if (wave == 0) {
@@ -132,17 +124,7 @@ prefill_f32_kernel(const float* __restrict__ q, int64_t q_sb, int64_t q_st, int6
                     sm.ent[n + __popcll(bal & ((1ull << lane) - 1ull))] = static_cast<uint32_t>(j) << 16 | mk;
                 n += __popcll(bal);
             }
-            if (lane == 0) {
-                // repeats after the union, in an order of their own (not of arrival)
-                const int nd = sm.n_dup;
-                for (int i = 0; i < nd; ++i) {
-                    const uint32_t x = sm.dup[i];
-                    int p = n + i;
-                    for (; p > n && sm.ent[p - 1] > x; --p) sm.ent[p] = sm.ent[p - 1];
-                    sm.ent[p] = x;
-                }
-                sm.n_ent = n + nd;
-            }
+            if (lane == 0) sm.n_ent = n;
         }
         __syncthreads();
         n_ent = sm.n_ent;
@@ -318,11 +300,12 @@ prefill_f32_kernel(const float* __restrict__ q, int64_t q_sb, int64_t q_st, int6
 }
 
 bool prefill_f32_supported(int dtype, int64_t T, int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int64_t B,
-                           const int32_t* sel, int64_t q_sb, int64_t q_st, int64_t q_sh, int64_t kv_sb,
+                           const int32_t* sel, int64_t cap, int64_t q_sb, int64_t q_st, int64_t q_sh, int64_t kv_sb,
                            int64_t kv_st, int64_t kv_sh, int64_t out_sb, int64_t out_st, const void* q,
                            const void* k, const void* v, const void* out) {
     if (dtype != SPARDA_F32 || D != 64 || (bs != 64 && bs != 32) || Hq % Hkv != 0 || Hq / Hkv > 16) return false;
-    if (sel != nullptr && cdiv(T, bs) > kFMaxNB) return false;
+    // a tile's list entries are counted in 32 bits, its blocks in the mask array
+    if (sel != nullptr && (cdiv(T, bs) > kFMaxNB || cap >= (int64_t(1) << 27))) return false;
     if (B * Hkv * cdiv(T, 16 / (Hq / Hkv)) >= (int64_t(1) << 31)) return false;
     if (kv_st >= (int64_t(1) << 22)) return false;  // offsets inside a block are 32-bit
     auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };

@@ -1,8 +1,6 @@
 """The fp32 matrix-core prefill (D = 64): group sizes, ragged tiles and blocks,
-dense and listed, causal and not, against the float64 oracle (max-abs 1e-4, the
-fp32 bar); lists with repeats, and infinite or NaN values of V that a token does
-not attend, against the general kernel (reached through a block size of 16 and
-through the token's own keys)."""
+dense and listed, causal and not, lists with repeats against the float64 oracle (max-abs 1e-4, the
+fp32 bar); infinite or NaN values of V that a token does not attend."""
 
 import numpy as np
 import pytest
@@ -35,22 +33,22 @@ def test_f32_prefill_against_the_oracle(R, T, bs, k, causal, dense):
     assert_close_out(np32(out), want, torch.float32)
 
 
-def test_f32_prefill_repeated_and_out_of_range_entries():
-    # a block of 64 keys listed twice = its four blocks of 16 keys listed twice
-    print("[case] f32 repeats", flush=True)
+@pytest.mark.parametrize("bs,R,cap", [
+    (64, 3, 3), (64, 1, 40), (64, 3, 112), (32, 16, 700)])  # every entry of a wide list in use
+def test_f32_prefill_repeated_and_out_of_range_entries(bs, R, cap):
+    # the allowed keys are a set: a repeat counts once, an entry outside the blocks not at all
+    print(f"[case] f32 repeats bs={bs} R={R} cap={cap}", flush=True)
     T, Hkv = 260, 2
-    x = synth.prefill_inputs(1, T, 6, Hkv, 64, dtype=torch.float32, seed=4)
-    d = {n: t.to(DEV) for n, t in x.items()}
+    x = synth.prefill_inputs(1, T, R * Hkv, Hkv, 64, dtype=torch.float32, seed=4)
     r = np.random.default_rng(5)
-    sel = np.stack([r.integers(-1, 6, (1, Hkv, T)) for _ in range(3)], -1).astype(np.int32)
+    sel = r.integers(-1, (T + bs - 1) // bs + 1, (1, Hkv, T, cap)).astype(np.int32)
     sel[..., 0] = 0
     sel[..., 2] = np.where(r.random((1, Hkv, T)) < 0.5, sel[..., 1], sel[..., 2])
-    n = r.integers(1, 4, (1, Hkv, T)).astype(np.int32)
-    fine = np.where(sel[..., None] >= 0, 4 * sel[..., None] + np.arange(4), -1).reshape(1, Hkv, T, 12).astype(np.int32)
-    to = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
-    got = sparda.prefill(d["q"], d["k"], d["v"], to(sel), to(n), 64)
-    want = sparda.prefill(d["q"], d["k"], d["v"], to(fine), to(4 * n), 16)
-    assert (got - want).abs().max().item() < 1e-5
+    n = r.integers(1, 4, (1, Hkv, T)).astype(np.int32) if cap == 3 else np.full((1, Hkv, T), cap, np.int32)
+    q, k, v, s_d, n_d = (t.to(DEV) for t in (x["q"], x["k"], x["v"], torch.from_numpy(sel), torch.from_numpy(n)))
+    got = sparda.prefill(q, k, v, s_d, n_d, bs)
+    want, _ = O.attention_prefill_masked(np32(x["q"]), np32(x["k"]), np32(x["v"]), sel, n, bs)  # lists as sets
+    assert_close_out(np32(got), want, torch.float32)
 
 
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
