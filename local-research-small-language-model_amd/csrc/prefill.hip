@@ -18,7 +18,7 @@ constexpr int kPrefillThreads = 256;
 constexpr int kPrefillWaves = kPrefillThreads / kWave;
 constexpr int kPrefillMaxGroup = 16;
 
-template <int DT, int DH>
+template <int DT, int DH, bool LISTED>
 __global__ void __launch_bounds__(kPrefillThreads)
 prefill_general_kernel(const void* __restrict__ q, int64_t q_sb, int64_t q_st, int64_t q_sh,
                        const void* __restrict__ k, const void* __restrict__ v,
@@ -43,7 +43,7 @@ prefill_general_kernel(const void* __restrict__ q, int64_t q_sb, int64_t q_st, i
     const int64_t limit = causal ? t + 1 : T;  // keys [0, limit)
 
     int n;
-    if (sel == nullptr) {
+    if constexpr (!LISTED) {
         n = static_cast<int>(causal ? t / bs + 1 : NB);
     } else {
         n = n_sel[row] < cap ? n_sel[row] : static_cast<int>(cap);
@@ -59,9 +59,27 @@ prefill_general_kernel(const void* __restrict__ q, int64_t q_sb, int64_t q_st, i
 #pragma unroll
     for (int r = 0; r < MAXR; ++r) acc[r].init();
 
+    // entries that repeat an earlier one are left out: bit i for the list's first 64, found in lanes
+    const int32_t* list = sel + row * cap;
+    uint64_t repeats = 0;
+    if constexpr (LISTED) {
+        const int mine = lane < n ? list[lane] : -1;
+        for (int i = 1; i < n && i < kWave; ++i)
+            if (__ballot(lane < i && mine == __builtin_amdgcn_readlane(mine, i)) != 0ull) repeats |= 1ull << i;
+    }
+    auto repeated = [&](int i, int j) {  // wave-uniform
+        if (i < kWave) return (repeats >> i & 1) != 0;
+        bool hit = false;
+        for (int e = lane; e < i; e += kWave) hit = hit || list[e] == j;
+        return __ballot(hit) != 0ull;
+    };
+
     for (int i = 0; i < n; ++i) {
-        const int64_t j = sel == nullptr ? i : sel[row * cap + i];
-        if (j < 0 || j >= NB) continue;
+        int64_t j = i;
+        if constexpr (LISTED) {
+            j = list[i];
+            if (j < 0 || j >= NB || repeated(i, static_cast<int>(j))) continue;
+        }
         const int64_t s0 = j * bs;
         int64_t s1 = s0 + bs;
         if (s1 > limit) s1 = limit;
@@ -355,7 +373,10 @@ int launch_prefill(const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh, cons
     dim3 grid(static_cast<unsigned>(T), static_cast<unsigned>(Hkv), static_cast<unsigned>(B));
     const float sl = scale * kLog2eP;
 #define SPARDA_PF(DT_, DH_)                                                                          \
-    hipLaunchKernelGGL((prefill_general_kernel<DT_, DH_>), grid, dim3(kPrefillThreads), 0, stream, q, \
+    if (sel != nullptr) SPARDA_PFL(DT_, DH_, true);                                                  \
+    else SPARDA_PFL(DT_, DH_, false)
+#define SPARDA_PFL(DT_, DH_, LISTED_)                                                                \
+    hipLaunchKernelGGL((prefill_general_kernel<DT_, DH_, LISTED_>), grid, dim3(kPrefillThreads), 0, stream, q, \
                        q_sb, q_st, q_sh, k, v, kv_sb, kv_st, kv_sh, sel, n_sel, cap, T,              \
                        static_cast<int>(Hq), static_cast<int>(Hkv), static_cast<int>(bs), causal, sl, \
                        out, out_sb, out_st)
@@ -373,6 +394,7 @@ int launch_prefill(const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh, cons
     }
 #undef SPARDA_PF_D
 #undef SPARDA_PF
+#undef SPARDA_PFL
     return check_hip(hipGetLastError(), "prefill_general_kernel");
 }
 

@@ -1,5 +1,6 @@
 """The fp32 matrix-core prefill (D = 64): group sizes, ragged tiles and blocks,
-dense and listed, causal and not, lists with repeats against the float64 oracle (max-abs 1e-4, the
+dense and listed, causal and not, lists with repeats (also on the general kernel,
+reached through a block size of 16) against the float64 oracle (max-abs 1e-4, the
 fp32 bar); infinite or NaN values of V that a token does not attend."""
 
 import numpy as np
@@ -34,7 +35,9 @@ def test_f32_prefill_against_the_oracle(R, T, bs, k, causal, dense):
 
 
 @pytest.mark.parametrize("bs,R,cap", [
-    (64, 3, 3), (64, 1, 40), (64, 3, 112), (32, 16, 700)])  # every entry of a wide list in use
+    (64, 3, 3), (16, 3, 3),                       # matrix-core and general kernel
+    (64, 1, 40), (64, 3, 112), (32, 16, 700),     # every entry of a wide list in use
+    (16, 2, 150)])
 def test_f32_prefill_repeated_and_out_of_range_entries(bs, R, cap):
     # the allowed keys are a set: a repeat counts once, an entry outside the blocks not at all
     print(f"[case] f32 repeats bs={bs} R={R} cap={cap}", flush=True)
