@@ -307,7 +307,7 @@ bool prefill_f32_supported(int dtype, int64_t T, int64_t Hq, int64_t Hkv, int64_
     // a tile's list entries are counted in 32 bits, its blocks in the mask array
     if (sel != nullptr && (cdiv(T, bs) > kFMaxNB || cap >= (int64_t(1) << 27))) return false;
     if (B * Hkv * cdiv(T, 16 / (Hq / Hkv)) >= (int64_t(1) << 31)) return false;
-    if (kv_st >= (int64_t(1) << 22)) return false;  // offsets inside a block are 32-bit
+    if (kv_st < 0 || kv_st >= (int64_t(1) << 22)) return false;  // offsets inside a block are 32-bit, unsigned
     auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     if (!al16(q) || !al16(k) || !al16(v) || !al16(out)) return false;
     return q_sb % 4 == 0 && q_st % 4 == 0 && q_sh % 4 == 0 && kv_sb % 4 == 0 && kv_st % 4 == 0 && kv_sh % 4 == 0 &&

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import sparda
-from sparda import synth
+from sparda import _lib, synth
 from oracle import sparda_oracle as O
 from helpers import assert_close_out, np32
 
@@ -52,6 +52,21 @@ def test_f32_prefill_repeated_and_out_of_range_entries(bs, R, cap):
     got = sparda.prefill(q, k, v, s_d, n_d, bs)
     want, _ = O.attention_prefill_masked(np32(x["q"]), np32(x["k"]), np32(x["v"]), sel, n, bs)  # lists as sets
     assert_close_out(np32(got), want, torch.float32)
+
+
+def test_f32_prefill_rows_in_descending_order():
+    # a negative token stride of K and V at the C entry (the first row is the last in memory)
+    print("[case] f32 negative stride", flush=True)
+    T, Hq, Hkv = 130, 6, 2
+    x = {n: t.to(DEV) for n, t in synth.prefill_inputs(1, T, Hq, Hkv, 64, dtype=torch.float32, seed=9).items()}
+    want = sparda.prefill(x["q"], x["k"], x["v"], None, None, 64)
+    q, k, v = x["q"], x["k"].flip(1).contiguous(), x["v"].flip(1).contiguous()
+    st, out = Hkv * 64, torch.empty_like(want)
+    end = 4 * st * (T - 1)
+    _lib.call("sparda_prefill", q.data_ptr(), *q.stride()[:3], k.data_ptr() + end, v.data_ptr() + end, T * st, -st, 64,
+              _lib.F32, None, None, 0, 1, T, Hq, Hkv, 64, 64, 1, 0.125, out.data_ptr(), *out.stride()[:2],
+              torch.cuda.current_stream().cuda_stream)
+    assert (out - want).abs().max().item() < 1e-5
 
 
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
