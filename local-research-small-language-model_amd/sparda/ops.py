@@ -234,7 +234,7 @@ def prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sel: Optional[tor
     ``select_fixed`` ([B,Hkv,T,cap] / [B,Hkv,T]) or None for dense.
     Returns out [B,T,Hq*D] in q's dtype.
     """
-    if sel is None and out is None:
+    if sel is None and n_sel is None and out is None:
         r = _host.prefill(q, k, v, block_size, causal, scale)
         if r is not None:
             return r if type(r) is not int else _lib.fail("sparda_prefill", r)
@@ -586,7 +586,7 @@ def decode_selected(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, S: int, b
     sel[b,g,i]. sel=None: dense over [0, S). k_new/v_new [B,Hkv,D]: the key and
     value of position S-1 (overriding what k/v hold there).
     """
-    if sel is None and out is None and k_new is None and v_new is None and not compact:
+    if sel is None and n_sel is None and out is None and k_new is None and v_new is None and not compact:
         r = _host.decode_dense(q, k, v, S, block_size, scale)
         if r is not None:
             return r if type(r) is not int else _lib.fail("sparda_decode_selected", r)

@@ -109,11 +109,14 @@ def test_refused_calls_raise_the_same(monkeypatch):
     q, k, v, f = x["q"], x["k"], x["v"], x["forecast"]
     protos = sparda.compress(k, 64)
     ids = torch.zeros(1, 130, 4, 64, dtype=torch.int32, device=DEV)
+    n = torch.ones(1, 4, 130, dtype=torch.int32, device=DEV)
     calls = [lambda: sparda.compress(k, 0), lambda: sparda.compress(ids, 64), lambda: sparda.compress(k.cpu(), 64),
              lambda: sparda.compress(k[0], 64), lambda: sparda.route(f, protos[:, :, :2], 64, 8),
              lambda: sparda.prefill(q, k.float(), v, None, None, 64), lambda: sparda.prefill(q[:, :, :11], k, v, None, None, 64),
              lambda: sparda.prefill_routed(q, k, v, f, protos, 32, 8), lambda: sparda.prefill_chunked(q, k, v, ids, 64, 8),
              lambda: sparda.decode_selected(q[:, 0], k, v, 131, 64), lambda: sparda.teacher_block_mass(q, k, 32),
+             lambda: sparda.prefill(q, k, v, None, n, 64),
+             lambda: sparda.decode_selected(q[:, 0], k, v, 130, 64, n_sel=n[:, :, 0]),
              lambda: sparda.ffn_decode(q, q, q, 1e-5), lambda: sparda.compress(k.requires_grad_(), 64)]
     for i, c in enumerate(calls):
         seen = []
