@@ -482,9 +482,8 @@ decode_attend_kernel(const void* __restrict__ q, int64_t q_sb, int64_t q_sh,
                     for (int i = 0; i < 4; ++i)
                         if (16 * nn + 4 * grp + i >= nk) sc[nn][i] = -__builtin_inff();
             }
-            float mx = max_sub_nn(sc);
-            mx = pair32_max(pair16_max(mx));
-            const float cand = mx * scale_log2;
+            // NaN where a score is: the reference then stays and the row sum is NaN
+            const float cand = pair32_max(pair16_max(max_acc(sc, -__builtin_inff()))) * scale_log2;
             const float m_new = cand > m_run + kLazy ? cand : m_run;
             const float alpha = m_new != m_run ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
             m_run = m_new;

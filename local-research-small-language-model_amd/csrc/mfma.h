@@ -26,39 +26,10 @@ __device__ __forceinline__ i16x4 lds_read_tr(const uint16_t* p) {
         (__attribute__((address_space(3))) i16x4*)(const_cast<uint16_t*>(p)));
 }
 
-// Reductions over lane pairs (l, l^16) and (l, l^32) with the gfx950 VALU
-// row swaps: permlane16_swap(x, x) hands every lane the values of rows
-// {2r, 2r+1} at its column, permlane32_swap(x, x) those of rows {r, r+2};
-// both lanes of a pair combine the same two values in the same order.
-// Maxima of values that are never NaN (attention scores: finite, or -inf where
-// masked). fmaxf in IEEE mode adds a quieting max per operand; these issue
-// v_max3_f32 / v_max_f32 as is.
-__device__ __forceinline__ float max3_nn(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-__device__ __forceinline__ float max_nn(float a, float b) {
-    float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-// max of the 16 accumulator values s[0..3][0..3]: 8 instructions
-__device__ __forceinline__ float max16_nn(const f32x4 (&s)[4]) {
-    const float a = max3_nn(s[0][0], s[0][1], s[0][2]);
-    const float b = max3_nn(s[0][3], s[1][0], s[1][1]);
-    const float c = max3_nn(s[1][2], s[1][3], s[2][0]);
-    const float d = max3_nn(s[2][1], s[2][2], s[2][3]);
-    const float e = max3_nn(s[3][0], s[3][1], s[3][2]);
-    return max_nn(max3_nn(a, b, c), max3_nn(d, e, s[3][3]));
-}
-// max of the 8 accumulator values s[0..1][0..3] (a 32-key block): 4 instructions
-__device__ __forceinline__ float max8_nn(const f32x4 (&s)[2]) {
-    return max_nn(max3_nn(max3_nn(s[0][0], s[0][1], s[0][2]), max3_nn(s[0][3], s[1][0], s[1][1]), s[1][2]), s[1][3]);
-}
 // max of m and 4 N accumulator values straight from the matrix cores, as
 // compiler-visible instructions (v_maximum3_f32), so that the wait states a
-// matrix result needs before a VALU reads it are placed by the compiler
+// matrix result needs before a VALU reads it are placed by the compiler (for
+// inline assembly it places none). A NaN among them gives NaN.
 template <int N>
 __device__ __forceinline__ float max_acc(const f32x4 (&s)[N], float m) {
 #pragma unroll
@@ -68,10 +39,10 @@ __device__ __forceinline__ float max_acc(const f32x4 (&s)[N], float m) {
     }
     return m;
 }
-// the maximum of a lane's scores of one block: 4 sub-tiles of 16 keys (64-key
-// block) or 2 (32-key block)
-__device__ __forceinline__ float max_sub_nn(const f32x4 (&s)[4]) { return max16_nn(s); }
-__device__ __forceinline__ float max_sub_nn(const f32x4 (&s)[2]) { return max8_nn(s); }
+// Reductions over lane pairs (l, l^16) and (l, l^32) with the gfx950 VALU
+// row swaps: permlane16_swap(x, x) hands every lane the values of rows
+// {2r, 2r+1} at its column, permlane32_swap(x, x) those of rows {r, r+2};
+// both lanes of a pair combine the same two values in the same order.
 // max with the lane 16 (SWAP16) or 32 lanes away. One asm block: a VALU write
 // of a register needs two wait states before a permlane swap reads it, and the
 // compiler does not count inline-assembly results as VALU writes, so the copy,

@@ -590,7 +590,7 @@ prefill_compact_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_s
 #pragma unroll
             for (int t = 0; t < kCChunk; ++t) {
                 if (t < nt) {
-                    const float cm = pair32_max(pair16_max(max_sub_nn(s[t]))) * scale_log2;
+                    const float cm = pair32_max(pair16_max(max_acc(s[t], -__builtin_inff()))) * scale_log2;
                     if (own[t]) atomicMax(reinterpret_cast<uint32_t*>(sm.lsum) + sl[t].c, order_key(cm));
                 }
             }

@@ -278,7 +278,7 @@ prefill_mfma_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, 
                     for (int i = 0; i < 4; ++i)
                         if (16 * n + 4 * grp + i > l) s[n][i] = -__builtin_inff();
             }
-            float mx = max16_nn(s);
+            float mx = max_acc(s, -__builtin_inff());
             mx = member[tt] ? mx : -__builtin_inff();
             mx = pair32_max(pair16_max(mx));
             const float cand = mx * scale_log2;  // this block's column max, log2 units
