@@ -20,8 +20,8 @@
 // kTGuard (a score far above block 0's, whose exponent would cost precision)
 // has the workgroup take the exact column maxima and walk again. The 4
 // lane groups' partial sums of a column are added by one fp32 matrix product
-// with a selector (v_mfma_f32_16x16x4_f32, exact products with 1 and 0). Windows
-// of more than kTKeep blocks do not keep every block sum: they walk once for the
+// with ones (v_mfma_f32_16x16x4_f32, exact products) per tile, whose results hold
+// their own column only (an infinite or NaN row stays alone). Windows of more than kTKeep blocks do not keep every block sum: they walk once for the
 // row sums alone and again for the block sums, written kTKeep blocks at a time.
 // B=4, T=4096, 12/4 heads: 105 us (490 TFLOP/s), from 205 us with two walks that both
 // exponentiated, a running maximum and lane-pair sums per block; B=1, T=8192
@@ -109,11 +109,6 @@ teacher_mass_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, 
 #pragma unroll
     for (int tt = 0; tt < R; ++tt) m[tt] = -__builtin_inff();
     float l = 0.0f;   // row sum of column col16 of tile grp (lanes with grp < R)
-    // selectors: product t adds tile t's four lane-group partials into row 4t of
-    // the result, element 0 of lane group t
-    float pick[R];
-#pragma unroll
-    for (int tt = 0; tt < R; ++tt) pick[tt] = col16 == 4 * tt ? 1.0f : 0.0f;
 
     // S^T of block j for every tile; masked keys at -inf
     const int64_t w_first = t0 + 16 * wave;
@@ -198,7 +193,7 @@ teacher_mass_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, 
                     for (int tt = 0; tt < R; ++tt)
                         m[tt] = pair32_max(pair16_max(max_acc(s[tt], -__builtin_inff()))) * scale_log2;
                 }
-                f32x4 d{0.f, 0.f, 0.f, 0.f};
+                float d = 0.0f;  // column col16 of tile grp
 #pragma unroll
                 for (int tt = 0; tt < R; ++tt) {
                     float a[4];
@@ -209,11 +204,14 @@ teacher_mass_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, 
                         for (int i = 1; i < 4; ++i)
                             a[n] += __builtin_amdgcn_exp2f(__builtin_fmaf(s[tt][n][i], scale_log2, -m[tt]));
                     }
-                    d = __builtin_amdgcn_mfma_f32_16x16x4f32(pick[tt], (a[0] + a[1]) + (a[2] + a[3]), d, 0, 0, 0);
+                    // the four lane groups' parts added: every row of the product is its column's sum, of that column alone
+                    const f32x4 c = __builtin_amdgcn_mfma_f32_16x16x4f32(1.0f, (a[0] + a[1]) + (a[2] + a[3]),
+                                                                         f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    d = tt == 0 || grp == tt ? c[0] : d;
                 }
-                if (count) l += d[0];
+                if (count) l += d;
                 if (store) {
-                    if (lane < 16 * R) ws[(j - j0) * kTSRow + lane] = d[0];
+                    if (lane < 16 * R) ws[(j - j0) * kTSRow + lane] = d;
                     if (!once && j - j0 == kTKeep - 1) {  // wave-uniform
                         flush(j0, j + 1);
                         j0 = j + 1;

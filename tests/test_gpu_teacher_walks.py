@@ -1,7 +1,8 @@
 """The teacher block mass over its workgroup shapes and walks: window edges,
 more blocks than a window keeps (row sums first, block sums in parts), and
 a score far above block 0's (the exact maxima and a second walk). fp32 sums of
-at most T terms: 1e-6 per probability against float64."""
+at most T terms: 1e-6 per probability against float64. Infinite and NaN elements
+stay with their own rows."""
 
 import numpy as np
 import pytest
@@ -32,3 +33,19 @@ def test_teacher_mass_shapes(B, T, Hq, Hkv, causal, hot):
     want = O.teacher_block_mass(np32(q[-1:]), np32(k[-1:]), 64, causal)
     assert np.abs(got[-1:] - want).max() < 1e-6 * (4 if hot else 1)
     assert np.abs(got.sum(-1) - 1.0).max() < 1e-5
+
+
+@pytest.mark.parametrize("R", [1, 2, 3])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+def test_teacher_mass_bad_elements_stay_in_their_rows(R, bad):
+    print(f"[case] teacher R={R} element {bad}", flush=True)
+    T, row, key = 200, 37, 150
+    g = torch.Generator().manual_seed(9)
+    q, k = torch.randn(1, T, R, 64, generator=g), torch.randn(1, T, 1, 64, generator=g)
+    q, k = q.to(torch.bfloat16), k.to(torch.bfloat16)
+    want = sparda.teacher_block_mass(q.to(DEV), k.to(DEV), 64).cpu().numpy()
+    q[0, row, 0, 5], k[0, key, 0, 7] = bad, bad
+    got = sparda.teacher_block_mass(q.to(DEV), k.to(DEV), 64).cpu().numpy()
+    clean = [t for t in range(key) if t != row]  # rows before the key, but the one
+    assert np.abs(got[:, :, clean] - want[:, :, clean]).max() < 1e-6
+    assert np.isnan(got[0, 0, row]).any()
