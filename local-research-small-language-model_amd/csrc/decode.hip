@@ -487,14 +487,15 @@ decode_attend_kernel(const void* __restrict__ q, int64_t q_sb, int64_t q_sh,
             const float m_new = cand > m_run + kLazy ? cand : m_run;
             const float alpha = m_new != m_run ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
             m_run = m_new;
+            const float neg = m_new == -__builtin_inff() ? -__builtin_inff() : -m_new;  // no score above -inf yet: P = 0
             uint4 pw[kHalf];
 #pragma unroll
             for (int mm = 0; mm < kHalf; ++mm) {
                 bf16x8 pb;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    pb[i] = static_cast<__bf16>(__builtin_amdgcn_exp2f(__builtin_fmaf(sc[2 * mm][i], scale_log2, -m_new)));
-                    pb[4 + i] = static_cast<__bf16>(__builtin_amdgcn_exp2f(__builtin_fmaf(sc[2 * mm + 1][i], scale_log2, -m_new)));
+                    pb[i] = static_cast<__bf16>(__builtin_amdgcn_exp2f(__builtin_fmaf(sc[2 * mm][i], scale_log2, neg)));
+                    pb[4 + i] = static_cast<__bf16>(__builtin_amdgcn_exp2f(__builtin_fmaf(sc[2 * mm + 1][i], scale_log2, neg)));
                 }
                 pw[mm] = __builtin_bit_cast(uint4, pb);
             }
@@ -700,7 +701,7 @@ decode_attend_kernel(const void* __restrict__ q, int64_t q_sb, int64_t q_sh,
         float num = 0.0f, den = 0.0f;
         for (int w = 0; w < nw; ++w) {
             const float* ps = part_all + (w * R + hh) * (DH + 2);
-            const float wt = __builtin_amdgcn_exp2f(ps[0] - M);
+            const float wt = ps[0] == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(ps[0] - M);
             den = den + wt * ps[1];
             num = num + wt * ps[2 + d];
         }
