@@ -9,10 +9,12 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 
 # SPARDA_LIBRARY overrides the path (an alternative build of the same ABI)
 LIB_PATH = os.environ.get("SPARDA_LIBRARY") or os.path.join(os.path.dirname(os.path.abspath(__file__)),
                                                             "libsparda.so")
+HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_host.so")
 
 F32 = 0
 BF16 = 1
@@ -190,10 +192,16 @@ class _NoHost:
 
 
 def load_host():
-    """The native host path (sparda._host) bound to the loaded library."""
+    """The native host path (sparda._host) bound to the loaded library. A module
+    that was not built is left out; one that is there and does not import (built
+    for another Python or torch) is reported."""
+    if not os.path.exists(HOST_PATH):
+        return _NoHost()
     try:
         from . import _host
-    except ImportError:
+    except ImportError as e:
+        warnings.warn(f"sparda: {HOST_PATH} cannot be imported, operators will call through Python "
+                      f"(build it again): {e}", RuntimeWarning)
         return _NoHost()
     import torch
 
