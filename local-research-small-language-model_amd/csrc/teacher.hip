@@ -13,19 +13,22 @@
 // LDS (double-buffered, the next block in flight in registers) and shared by
 // the wavefronts; S^T = K Q^T per block and tile with v_mfma_f32_16x16x32_bf16.
 // Bound by the exponentials and the matrix products of the scores, so each score
-// is formed and exponentiated once: against the column's maximum over block 0
-// (which every column attends, key 0 being allowed to every token), the block
-// sums fp32 per column in LDS, and with them the row sums; the window's rows are
-// normalised and written at the end, coalesced along the blocks. A row sum past
-// kTGuard (a score far above block 0's, whose exponent would cost precision)
-// has the workgroup take the exact column maxima and walk again. The 4
-// lane groups' partial sums of a column are added by one fp32 matrix product
-// with ones (v_mfma_f32_16x16x4_f32, exact products) per tile, whose results hold
-// their own column only (an infinite or NaN row stays alone). Windows of more than kTKeep blocks do not keep every block sum: they walk once for the
-// row sums alone and again for the block sums, written kTKeep blocks at a time.
-// B=4, T=4096, 12/4 heads: 105 us (490 TFLOP/s), from 205 us with two walks that both
-// exponentiated, a running maximum and lane-pair sums per block; B=1, T=8192
-// (two walks) 249 us, from 325.
+// is formed and exponentiated once: against the column's reference, its maximum
+// over block 0 (which every column attends, key 0 being allowed to every token),
+// the block sums fp32 per column in LDS, and with them the row sums; the window's
+// rows are normalised and written at the end, coalesced along the blocks. Where a
+// score lies so far above the reference that its exponent would cost precision
+// (kTGuard), the wavefront raises its references to the block's maxima, scales
+// what it holds and forms that block's sums again: one walk whatever the scores
+// are. The 4 lane groups' partial sums of a column are added by one fp32 matrix
+// product with ones (v_mfma_f32_16x16x4_f32, exact products) per tile, whose
+// results hold their own column only (an infinite or NaN row stays alone). Windows
+// of more than kTKeep blocks do not keep every block sum: they walk once for the
+// row sums and references and again for the block sums, written kTKeep blocks at a time.
+// B=4, T=4096, 12/4 heads: 106 us (485 TFLOP/s), 119 with a raise in every window
+// (scores that peak at the token itself); 204 with two walks that both
+// exponentiated, a running maximum and lane-pair sums per block. B=1, T=8192 (two
+// walks) 253 us, from 325.
 #include "common.h"
 #include "kernels.h"
 #include "mfma.h"
@@ -37,7 +40,7 @@ constexpr int kTD = 64;            // head dim
 constexpr int kTKRow = kTD + 8;    // K row in LDS (bf16 elements, 144 B)
 constexpr int kTKeep = 64;         // block sums kept per column (50 KB of LDS for 4 wavefronts, two workgroups per CU)
 constexpr int kTSRow = 49;         // LDS row of one block's column sums (odd: reads along the blocks are conflict-free)
-constexpr float kTGuard = 65536.0f; // 2^16
+constexpr float kTGuard = 16384.0f; // 2^14: a lane's part of a block sum past it raises the references
 constexpr int64_t kTCus = 256;
 
 template <int R, int NW>
@@ -51,7 +54,6 @@ teacher_mass_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, 
     constexpr int kWin = 16 * NW;                // tokens per workgroup
     constexpr int kCh = kTBs * 8 / kThreads;     // 16-byte K chunks each thread stages per block
     __shared__ uint16_t kst[2][kTBs * kTKRow];
-    __shared__ int flag;                         // some row sum passed kTGuard
     extern __shared__ float sums[];              // [NW][min(NB, kTKeep)][kTSRow]
     const int tid = threadIdx.x;
     const int lane = tid % kWave;
@@ -106,9 +108,7 @@ teacher_mass_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, 
     };
 
     float m[R];     // the columns' references (log2 units)
-#pragma unroll
-    for (int tt = 0; tt < R; ++tt) m[tt] = -__builtin_inff();
-    float l = 0.0f;   // row sum of column col16 of tile grp (lanes with grp < R)
+    float l = 0.0f; // row sum of column col16 of tile grp (lanes with grp < R)
 
     // S^T of block j for every tile; masked keys at -inf
     const int64_t w_first = t0 + 16 * wave;
@@ -169,53 +169,83 @@ teacher_mass_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, 
         __builtin_amdgcn_wave_barrier();
     };
 
-    // one pass over the blocks. maxima: the exact column maxima (lane-local) into
-    // m; else the block sums against m (set from block 0 unless `exact`): added
-    // into l (count) and kept, written when kTKeep of them are held (store)
-    auto walk = [&](bool maxima, bool exact, bool count, bool store) __attribute__((always_inline)) {
+    // this lane's part (16 keys) of the block sums of column col16 of each tile, from
+    // the scores against m; returns the largest
+    auto expsum = [&](const f32x4 (&s)[R][4], float (&part)[R]) __attribute__((always_inline)) {
+        float top = 0.0f;
+#pragma unroll
+        for (int tt = 0; tt < R; ++tt) {
+            float a[4];
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+                a[n] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[tt][n][0], scale_log2, -m[tt]));
+#pragma unroll
+                for (int i = 1; i < 4; ++i)
+                    a[n] += __builtin_amdgcn_exp2f(__builtin_fmaf(s[tt][n][i], scale_log2, -m[tt]));
+            }
+            part[tt] = (a[0] + a[1]) + (a[2] + a[3]);
+            top = __builtin_elementwise_maximum(top, part[tt]);
+        }
+        return top;
+    };
+
+    // one pass over the blocks: the block sums against m, added into l (count) and
+    // kept, written when kTKeep of them are held (store). The first walk (refs) sets m
+    // from block 0 and raises it where a lane's part of a later block's sum passes
+    // the guard; what is held by then is scaled to the new reference.
+    auto walk = [&](bool refs, bool count, bool store) __attribute__((always_inline)) {
         StageV nk{};
         fetch(0, nk);
         __syncthreads();  // the previous walk has read its last buffer
         stash(0, nk);
         if (jmax >= 1) fetch(1, nk);
         __syncthreads();
+        if (refs) {
+            f32x4 s[R][4];
+            scores(0, 0, s);
+#pragma unroll
+            for (int tt = 0; tt < R; ++tt) {
+                const float mx = pair32_max(pair16_max(max_acc(s[tt], -__builtin_inff()))) * scale_log2;
+                m[tt] = mx == -__builtin_inff() ? -__FLT_MAX__ : mx;  // a block of -inf scores: any later one is above
+            }
+        }
         int j0 = 0;  // first block held in `ws`
         for (int j = 0; j <= jmax; ++j) {
             const int buf = j & 1;
             f32x4 s[R][4];
             scores(buf, j, s);
-            if (maxima) {
-#pragma unroll
-                for (int tt = 0; tt < R; ++tt) m[tt] = max_acc(s[tt], m[tt]);
-            } else {
-                if (j == 0 && !exact) {  // wave-uniform
-#pragma unroll
-                    for (int tt = 0; tt < R; ++tt)
-                        m[tt] = pair32_max(pair16_max(max_acc(s[tt], -__builtin_inff()))) * scale_log2;
-                }
-                float d = 0.0f;  // column col16 of tile grp
+            float part[R];
+            const float top = expsum(s, part);
+            if (refs && __builtin_expect(__ballot(!(top <= kTGuard)) != 0ull, 0)) {  // wave-uniform
+                // raise the references to this block's maxima (not to a NaN)
+                float f = 1.0f;
 #pragma unroll
                 for (int tt = 0; tt < R; ++tt) {
-                    float a[4];
-#pragma unroll
-                    for (int n = 0; n < 4; ++n) {
-                        a[n] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[tt][n][0], scale_log2, -m[tt]));
-#pragma unroll
-                        for (int i = 1; i < 4; ++i)
-                            a[n] += __builtin_amdgcn_exp2f(__builtin_fmaf(s[tt][n][i], scale_log2, -m[tt]));
-                    }
-                    // the four lane groups' parts added: every row of the product is its column's sum, of that column alone
-                    const f32x4 c = __builtin_amdgcn_mfma_f32_16x16x4f32(1.0f, (a[0] + a[1]) + (a[2] + a[3]),
-                                                                         f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                    d = tt == 0 || grp == tt ? c[0] : d;
+                    const float mx = pair32_max(pair16_max(max_acc(s[tt], -__builtin_inff()))) * scale_log2;
+                    const bool up = mx > m[tt];
+                    const float ft = up ? __builtin_amdgcn_exp2f(m[tt] - mx) : 1.0f;
+                    m[tt] = up ? mx : m[tt];
+                    f = grp == tt ? ft : f;
                 }
-                if (count) l += d;
-                if (store) {
-                    if (lane < 16 * R) ws[(j - j0) * kTSRow + lane] = d;
-                    if (!once && j - j0 == kTKeep - 1) {  // wave-uniform
-                        flush(j0, j + 1);
-                        j0 = j + 1;
-                    }
+                l *= f;
+                if (store && lane < 16 * R)
+#pragma unroll 1
+                    for (int r = 0; r < j - j0; ++r) ws[r * kTSRow + lane] *= f;
+                expsum(s, part);
+            }
+            // the four lane groups' parts added: every row of the product is its column's sum, of that column alone
+            float d = 0.0f;  // column col16 of tile grp
+#pragma unroll
+            for (int tt = 0; tt < R; ++tt) {
+                const f32x4 c = __builtin_amdgcn_mfma_f32_16x16x4f32(1.0f, part[tt], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                d = tt == 0 || grp == tt ? c[0] : d;
+            }
+            if (count) l += d;
+            if (store) {
+                if (lane < 16 * R) ws[(j - j0) * kTSRow + lane] = d;
+                if (!once && j - j0 == kTKeep - 1) {  // wave-uniform
+                    flush(j0, j + 1);
+                    j0 = j + 1;
                 }
             }
             if (j + 1 <= jmax) {
@@ -224,24 +254,10 @@ teacher_mass_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, 
             }
             __syncthreads();
         }
-        if (store && !once) flush(j0, jmax + 1);
+        if (store && j0 <= jmax) flush(j0, jmax + 1);
     };
-    if (tid == 0) flag = 0;  // ordered before its uses by the walk's barriers
-    walk(false, false, true, once);
-    const bool bad = lane < 16 * R && !(l <= kTGuard);
-    if (__ballot(bad) != 0ull && lane == 0) atomicOr(&flag, 1);
-    __syncthreads();
-    if (flag != 0) {  // workgroup-uniform
-#pragma unroll
-        for (int tt = 0; tt < R; ++tt) m[tt] = -__builtin_inff();
-        walk(true, true, false, false);
-#pragma unroll
-        for (int tt = 0; tt < R; ++tt) m[tt] = pair32_max(pair16_max(m[tt])) * scale_log2;
-        l = 0.0f;
-        walk(false, true, true, once);
-    }
-    if (once) flush(0, jmax + 1);
-    else walk(false, true, false, true);
+    walk(true, true, once);
+    if (!once) walk(false, false, true);
     // blocks past the causal limit carry no probability
     if (jmax + 1 < NB) {
         for (int tk = 0; tk < 16; ++tk) {

@@ -1,8 +1,8 @@
 """The teacher block mass over its workgroup shapes and walks: window edges,
 more blocks than a window keeps (row sums first, block sums in parts), and
-a score far above block 0's (the exact maxima and a second walk). fp32 sums of
-at most T terms: 1e-6 per probability against float64. Infinite and NaN elements
-stay with their own rows."""
+scores far above those before (the reference raised, once and many times, and
+after a block of -inf scores). fp32 sums of at most T terms: 1e-6 per
+probability against float64. Infinite and NaN elements stay with their own rows."""
 
 import numpy as np
 import pytest
@@ -33,6 +33,23 @@ def test_teacher_mass_shapes(B, T, Hq, Hkv, causal, hot):
     want = O.teacher_block_mass(np32(q[-1:]), np32(k[-1:]), 64, causal)
     assert np.abs(got[-1:] - want).max() < 1e-6 * (4 if hot else 1)
     assert np.abs(got.sum(-1) - 1.0).max() < 1e-5
+
+
+@pytest.mark.parametrize("T,Hq,Hkv", [(500, 12, 4), (500, 4, 4), (4200, 2, 1)])
+def test_teacher_mass_rising_scores(T, Hq, Hkv):
+    # every row's scores rise by 24 log2-units from block to block of its last few: each raises the reference
+    print(f"[case] teacher rising T={T} Hq={Hq} Hkv={Hkv}", flush=True)
+    g = torch.Generator().manual_seed(T)
+    q, k = torch.randn(1, T, Hq, 64, generator=g), torch.randn(1, T, Hkv, 64, generator=g)
+    b = torch.arange(T) // 64
+    q[..., 0] = 8.0
+    k[..., 0] = (16.0 * torch.clamp(b - (T // 64 - 5), min=0)).to(torch.float32)[None, :, None]
+    k[:, :64, :, 0] = float("-inf")  # block 0: nothing
+    q, k = q.to(torch.bfloat16), k.to(torch.bfloat16)
+    got = sparda.teacher_block_mass(q.to(DEV), k.to(DEV), 64).cpu().numpy()
+    want = O.teacher_block_mass(np32(q), np32(k), 64, True)
+    assert np.abs(got[:, :, 64:] - want[:, :, 64:]).max() < 4e-6
+    assert np.isnan(got[:, :, :64, 0]).all()  # rows with no finite score
 
 
 @pytest.mark.parametrize("R", [1, 2, 3])
