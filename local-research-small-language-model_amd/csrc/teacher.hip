@@ -28,7 +28,7 @@
 // B=4, T=4096, 12/4 heads: 106 us (485 TFLOP/s), 119 with a raise in every window
 // (scores that peak at the token itself); 204 with two walks that both
 // exponentiated, a running maximum and lane-pair sums per block. B=1, T=8192 (two
-// walks) 253 us, from 325.
+// walks) 253 us, from 325; one block (T=64) 5.5 us.
 #include "common.h"
 #include "kernels.h"
 #include "mfma.h"
@@ -54,6 +54,7 @@ teacher_mass_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, 
     constexpr int kWin = 16 * NW;                // tokens per workgroup
     constexpr int kCh = kTBs * 8 / kThreads;     // 16-byte K chunks each thread stages per block
     __shared__ uint16_t kst[2][kTBs * kTKRow];
+    __shared__ float lrow[NW][16 * R];           // the columns' row sums
     extern __shared__ float sums[];              // [NW][min(NB, kTKeep)][kTSRow]
     const int tid = threadIdx.x;
     const int lane = tid % kWave;
@@ -146,25 +147,30 @@ teacher_mass_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, 
     const int keep = static_cast<int>(NB < kTKeep ? NB : kTKeep);
     const bool once = jmax < kTKeep;  // every block sum is kept: one walk
     float* ws = sums + static_cast<int64_t>(wave) * keep * kTSRow;
-    // normalises and writes blocks [j0, j1) of the wavefront's rows from `ws`
-    // (filled by this wavefront alone): lane -> block j0 + lane
+    // normalises and writes blocks [j0, j1) of the wavefront's rows from `ws` and
+    // `lrow` (filled by this wavefront alone): lanes along the blocks of a token,
+    // then its next tokens, so that few blocks do not leave lanes idle
     auto flush = [&](int j0, int j1) __attribute__((always_inline)) {
         __builtin_amdgcn_wave_barrier();
+        const int nb = j1 - j0;
+        int tk = lane / nb, jj = lane % nb;
+        const int dt = kWave / nb, dj = kWave % nb;
+        const int rows = static_cast<int>(T - w_first < 16 ? T - w_first : 16);
+        const int ld = static_cast<int>(NB);
+        float* out = mass + ((static_cast<int64_t>(b) * H + g) * T + w_first) * NB + j0;
+        const float* lr = lrow[wave];
 #pragma unroll 2
-        for (int tk = 0; tk < 16; ++tk) {
-            const int64_t t = w_first + tk;
-            if (t >= T) break;  // wave-uniform
+        for (int e = lane; e < 16 * nb; e += kWave) {
             float v = 0.0f;
-            const int row = j0 + lane < j1 ? lane : 0;
 #pragma unroll
-            for (int hh = 0; hh < R; ++hh) {
-                const int c = R * tk + hh;
-                // the column's row sum sits in lane c (tile c / 16, column c % 16)
-                const float lc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, l), c));
-                v += ws[row * kTSRow + c] / lc;
+            for (int hh = 0; hh < R; ++hh) v += ws[jj * kTSRow + R * tk + hh] / lr[R * tk + hh];
+            if (tk < rows) out[tk * ld + jj] = v / static_cast<float>(R);
+            tk += dt;
+            jj += dj;
+            if (jj >= nb) {
+                jj -= nb;
+                ++tk;
             }
-            if (j0 + lane < j1)
-                mass[((static_cast<int64_t>(b) * H + g) * T + t) * NB + j0 + lane] = v / static_cast<float>(R);
         }
         __builtin_amdgcn_wave_barrier();
     };
@@ -254,6 +260,7 @@ teacher_mass_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st, 
             }
             __syncthreads();
         }
+        if (count && lane < 16 * R) lrow[wave][lane] = l;
         if (store && j0 <= jmax) flush(j0, jmax + 1);
     };
     walk(true, true, once);
