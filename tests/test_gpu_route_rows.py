@@ -1,6 +1,7 @@
 """The router's matrix-core scores against the oracle's fma chain, bit for bit:
-row sets and block chunks at their edges, every forecast width, and forecasts
-with denormal, infinite and NaN elements."""
+row sets and block chunks at their edges, every forecast
+width, and forecasts with denormal, cancelling, infinite and NaN elements and of
+mixed magnitude (where a chain differs from any other order of the sum)."""
 
 import numpy as np
 import pytest
@@ -17,6 +18,7 @@ DEV = "cuda"
 @pytest.mark.parametrize("Tq,NB,Df,k,causal,kind", [
     (1, 1, 64, 1, True, "normal"), (63, 2, 16, 2, True, "normal"), (65, 15, 32, 8, False, "normal"),
     (129, 17, 64, 8, True, "normal"), (200, 33, 128, 16, False, "normal"), (1000, 49, 64, 32, True, "normal"),
+    (130, 70, 64, 8, False, "cancelling"), (130, 70, 128, 8, True, "mixed"), (130, 70, 16, 8, False, "mixed"),
     (130, 97, 64, 8, False, "tiny"), (130, 64, 64, 8, False, "infinite"), (130, 40, 64, 4, False, "equal")])
 def test_route_scores_and_lists(Tq, NB, Df, k, causal, kind):
     print(f"[case] route Tq={Tq} NB={NB} Df={Df} {kind}", flush=True)
@@ -26,6 +28,12 @@ def test_route_scores_and_lists(Tq, NB, Df, k, causal, kind):
     p = torch.randn(2, NB, H, Df, generator=g)
     if kind == "tiny":
         f, p = f * 1e-20, p * 1e-20      # scores around 1e-39: denormal
+    if kind == "cancelling":             # pairs of terms that leave a few bits, and sums that leave none
+        f[..., 1::2], p[..., 1::2] = f[..., ::2], -p[..., ::2] * (1 + 2.0 ** -14)
+        p[:, ::3, :, Df // 2:], f[..., Df // 2:] = -p[:, ::3, :, :Df // 2], f[..., :Df // 2]
+    if kind == "mixed":                  # terms of 2^-40 to 2^40
+        f = f * 2.0 ** torch.randint(-20, 21, f.shape, generator=g)
+        p = p * 2.0 ** torch.randint(-20, 21, p.shape, generator=g)
     if kind == "infinite":
         p[:, ::7, :, 5] = float("inf")   # scores +inf or -inf
     if kind == "equal":
