@@ -12,10 +12,12 @@
 // their group (double-buffered; the next block is loaded into registers while
 // the current one is computed) and shared by the window's tokens and R heads.
 // The groups share the columns' references, so their O and row sums are added
-// at the end, in group order. Small windows times key groups keep the number of
-// workgroups well past one per CU, so that the causal triangle balances: at B=1,
-// T=8192, 12/4 heads 128 us (800 TFLOP/s) against 231 with one group and 128-token
-// windows (256 workgroups, the heaviest twice the mean). Bound by issue: a wave's
+// at the end, in group order. Where windows are few, small ones times key groups
+// keep the number of workgroups well past one per CU, so that the causal triangle
+// balances: at B=1, T=8192, 12/4 heads 128 us (800 TFLOP/s) against 231 with one
+// group and 128-token windows (256 workgroups, the heaviest twice the mean); where
+// they are many, one group stages a block for the most tokens (the launcher's
+// rule, with its times). Bound by issue: a wave's
 // exponentials and products take turns, so that the matrix cores are busy about
 // 40% of the time. Per tile and block, with v_mfma_f32_16x16x32_bf16:
 //     S^T[key, col] = K[key, :] . Q[col, :]           (8 MFMA)
@@ -112,7 +114,8 @@ prefill_dense_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_st,
     // wave-uniform (scalar registers): the token wave, and the key group, which
     // walks the blocks kg, kg + KG, ...
     const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
-    const int wave = wv % CW, kg = wv / CW;
+    constexpr bool kOne = KG == 1 && !LISTED;  // (the listed form spills ten registers more with the index folded)
+    const int wave = kOne ? wv : wv % CW, kg = kOne ? 0 : wv / CW;
     const int tid = wave * kWave + lane;         // thread within its key group
     const int col16 = lane % 16;
     const int grp = lane / 16;
@@ -473,12 +476,34 @@ int launch_prefill_dense(const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh
                        static_cast<const uint16_t*>(v), kv_sb, kv_st, kv_sh, T, static_cast<int>(Hkv),     \
                        cdiv(T, 16 * CW_), causal, sl, static_cast<uint16_t*>(out), out_sb, out_st, ChunkArgs{})
 #define SPARDA_DN_W(R_)                         \
-    if (wide) SPARDA_DN(R_, 4, 2);              \
-    else SPARDA_DN(R_, 2, 4);
-    // 64-token windows from 5/4 workgroups per CU on, else 32-token windows of
-    // four key groups (12/4 heads: 49 us against 64 at T=4096, 256 windows of 64;
-    // 99 us against 91 at T=6000, 376 windows; 25 against 36 at T=2048)
-    const bool wide = 4 * B * Hkv * cdiv(T, 64) > 5 * kDCus;
+    if (groups == 4) SPARDA_DN(R_, 2, 4);       \
+    else if (groups == 2) SPARDA_DN(R_, 4, 2);  \
+    else SPARDA_DN(R_, 8, 1);
+    // Windows of 128 tokens stage a block for the most tokens, key groups cut a
+    // window's serial walk: groups where windows are few against the CUs and the
+    // walk is long. W 128-token windows of up to NB blocks; times in us of
+    // 1 / 2 / 4 groups, 12/4 heads, causal.
+    //  - one block: nothing to share (T=64, B=1: 7.8 / 9.3 / 9.1).
+    //  - up to a quarter of a window a CU: four groups (T=2048: 66 / 36 / 24; for
+    //    R = 4, whose four-group form spills, from 4 blocks on: B=16, T=128 14.0 /
+    //    12.6 / 14.9), up to half a window on long causal walks (T=4096: 125 / 64 / 48).
+    //  - past that the longest walk against the sum of all walks: one group takes
+    //    the time of NB blocks at W = 256, as many as W / 256 NB / 2 above, and two
+    //    groups half a walk and a fixed cost: they cross at NB = 12 (W / 256)^2
+    //    (W = 256: T=512 25 / 25, T=1024 39 / 32; W = 512: T=2048 82 / 85, T=4096
+    //    145 / 142) or 80 (W = 1024: T=4096 275 / 280, T=8192 514 / 500). With one or
+    //    two heads a tile's products hide less staging: not past 3/2 windows a CU
+    //    (8/4 heads, W = 512, T=2048: 59 / 67).
+    //  - without the mask every walk is the same: two groups up to half a window a
+    //    CU, or on long walks of three and four heads (B=4, T=3000: 187 / 149).
+    const int64_t NB = cdiv(T, kDBs);
+    const int64_t windows = B * Hkv * cdiv(T, 128), W = windows < (1 << 20) ? windows : (1 << 20);
+    const bool crossed = causal ? (NB * kDCus * kDCus >= 12 * W * W || NB >= 80) && (R >= 3 || 2 * W <= 3 * kDCus)
+                                : 2 * W <= kDCus || (R >= 3 && NB >= 24);
+    const int groups = NB == 1 ? 1
+                       : (R < 4 || NB >= 4) && (4 * W <= kDCus || (causal && 2 * W <= kDCus && NB >= 20)) ? 4
+                       : crossed ? 2
+                                 : 1;
     switch (R) {
         case 1: SPARDA_DN_W(1); break;
         case 2: SPARDA_DN_W(2); break;

@@ -1,6 +1,6 @@
-"""The dense prefill's workgroup shapes (64 tokens x 2 key groups, 32 tokens x 4):
+"""The dense prefill's workgroup shapes (128 tokens x 1 key group, 64 x 2, 32 x 4):
 lengths that leave key groups without a block, ragged windows and blocks, and
-the length where the shape changes, against the float64 oracle; and the exact
+the sizes where the shape changes, against the float64 oracle; and the exact
 walk of every group after a score far above block 0's."""
 
 import numpy as np
@@ -17,8 +17,11 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("R", [1, 3, 4])
-@pytest.mark.parametrize("B,T,causal", [(1, 31, True), (1, 33, False), (1, 193, True), (2, 321, False),
-                                        (1, 5121, True)])
+@pytest.mark.parametrize("B,T,causal", [
+    (1, 31, True), (1, 64, False), (1, 65, True),           # one block; two
+    (1, 193, True), (2, 321, False), (16, 100, True),       # four groups
+    (17, 193, True), (16, 250, False), (1, 5121, True),     # two
+    (43, 130, True), (33, 129, False), (65, 65, True)])     # more windows than CUs: one
 def test_dense_prefill_key_groups(R, B, T, causal):
     print(f"[case] dense groups R={R} B={B} T={T} causal={causal}", flush=True)
     x = synth.prefill_inputs(B, T, 4 * R, 4, 64, dtype=torch.bfloat16, seed=700 + T)
@@ -32,14 +35,16 @@ def test_dense_prefill_key_groups(R, B, T, causal):
     assert_close_out(np32(out), want, torch.bfloat16, mask)
 
 
-@pytest.mark.parametrize("hot_key", [70, 130, 200, 260])  # a block of each of four key groups
-def test_dense_prefill_exact_walk_over_every_key_group(hot_key):
-    print(f"[case] dense exact walk, hot key {hot_key}", flush=True)
-    x = synth.prefill_inputs(1, 320, 12, 4, 64, dtype=torch.float32, seed=95)
+@pytest.mark.parametrize("B,hot_key", [(1, 70), (1, 130), (1, 200), (1, 260),  # a block of each of four key groups
+                                       (6, 70), (6, 260), (14, 260)])         # of two, of one
+def test_dense_prefill_exact_walk_over_every_key_group(B, hot_key):
+    print(f"[case] dense exact walk, B={B} hot key {hot_key}", flush=True)
+    x = synth.prefill_inputs(B, 320, 12, 4, 64, dtype=torch.float32, seed=95)
     q, k, v = x["q"].clone(), x["k"].clone(), x["v"].clone()
     e = torch.zeros(64)
     e[0] = 20.0
     q[0, 300], k[0, 300], k[0, 0], k[0, hot_key] = e, -e, -e, e  # 72 log2-units above the other scores
     q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
     out = np32(sparda.prefill(q.to(DEV), k.to(DEV), v.to(DEV), None, None, 64))
-    assert_close_out(out, O.attention_prefill(np32(q), np32(k), np32(v), None, None, 64, True), torch.bfloat16)
+    assert_close_out(out[:1], O.attention_prefill(np32(q[:1]), np32(k[:1]), np32(v[:1]), None, None, 64, True),
+                     torch.bfloat16)
