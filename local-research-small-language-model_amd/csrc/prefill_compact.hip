@@ -218,7 +218,7 @@ prefill_compact_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_s
                           kRG * kCRouteK * W * sizeof(double) <= sizeof(sm.vstage),
                       "routing in the V staging bytes");
         KeyTopK<kCRouteK> best[kRT];
-        route_tiles<FDT, kCRouteDf, kCRouteK, kCWaves, kRP, kRG, kRT, 1>(
+        route_tiles<FDT, kCRouteDf, kCRouteK, kCWaves, kRP, kRG, kRT, 1, true>(
             rt.f, rt.fsb, rt.fst, rt.fsh, rt.protos, b, g, H, t0, W, T, NB, BS, causal, 0, rt.scale, nullptr,
             reinterpret_cast<float*>(&sm.vstage[0][0]), best);
         __syncthreads();  // the last prototypes have been read

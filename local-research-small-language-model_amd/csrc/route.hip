@@ -78,19 +78,20 @@ int launch_compress(const void* k, int dtype, int64_t B, int64_t S, int64_t H, i
 // router. Under the causal mask a workgroup of kRouteWaves wavefronts takes two
 // sets of 64 consecutive rows of one (b, h): set p and its mirror NS-1-p, so
 // that every workgroup scores about the same number of (row, block) pairs;
-// without it every set has the same work and a workgroup takes one. Within a
-// set every wavefront takes 16 rows and all candidate blocks, 32 at a time
-// (two independent product chains), staged once in LDS for the four of them
+// without it every set has the same work, and where sets are few a workgroup
+// takes one. Within a
+// set every wavefront takes 16 rows and all candidate blocks, 16 TB at a time
+// (TB independent product chains), staged once in LDS for the four of them
 // (route_tiles); its lanes 0..15 then write their rows' outputs.
 // ---------------------------------------------------------------------------
-template <int FDT, int DF, int KMAX>
+template <int FDT, int DF, int KMAX, int TB>
 __global__ void __launch_bounds__(kRouteThreads)
 route_rows_kernel(const void* __restrict__ f, int64_t fsb, int64_t fst, int64_t fsh,
                   const float* __restrict__ protos, int64_t Tq, int H, int64_t NB, int bs,
                   int ke, int causal, int64_t score_pos0, int64_t query_pos0, float scale,
                   int32_t* __restrict__ topk, float* __restrict__ scores,
                   int32_t* __restrict__ sel, int32_t* __restrict__ n_sel, int cap) {
-    using Shape = RouteShape<DF, kRouteWaves, kRouteWaves, 1, 1, 2>;
+    using Shape = RouteShape<DF, kRouteWaves, kRouteWaves, 1, 1, TB>;
     static_assert(Shape::kRows == kWave, "a set is 64 rows");
     __shared__ __attribute__((aligned(16))) float lds[Shape::kFloats];
     const int lane = threadIdx.x % kWave;
@@ -101,13 +102,14 @@ route_rows_kernel(const void* __restrict__ f, int64_t fsb, int64_t fst, int64_t 
     const int64_t pair = blockIdx.x;
 
     for (int pass = 0; pass < 2; ++pass) {
-        const int64_t set = pass == 0 ? pair : NS - 1 - pair;
-        if (pass == 1 && (!causal || set == pair)) break;  // one set without the mask; an odd count's middle set
+        const bool one = gridDim.x == NS;  // a set a workgroup, the heaviest first
+        const int64_t set = pass == 0 && !one ? pair : NS - 1 - pair;
+        if (pass == 1 && (one || set == pair)) break;  // an odd count's middle set
         KeyTopK<KMAX> best[1];
         __syncthreads();  // the previous set's last chunk has been read
-        route_tiles<FDT, DF, KMAX, kRouteWaves, kRouteWaves, 1, 1, 2>(f, fsb, fst, fsh, protos, b, h, H, set * kWave,
-                                                                      kWave, Tq, NB, bs, causal, score_pos0, scale,
-                                                                      scores, lds, best);
+        route_tiles<FDT, DF, KMAX, kRouteWaves, kRouteWaves, 1, 1, TB, false>(
+            f, fsb, fst, fsh, protos, b, h, H, set * kWave, kWave, Tq, NB, bs, causal, score_pos0, scale, scores, lds,
+            best);
         const int64_t t = set * kWave + 16 * wave + lane;
         if (lane >= 16 || t >= Tq) continue;
         int32_t picks[KMAX];
@@ -138,16 +140,27 @@ static int launch_route_df(const void* f, int64_t fsb, int64_t fst, int64_t fsh,
                            int causal, int64_t score_pos0, int64_t query_pos0, float scale,
                            int32_t* topk, float* scores, int32_t* sel, int32_t* n_sel, int cap,
                            hipStream_t stream) {
-    const int64_t pairs = causal ? cdiv(cdiv(Tq, kWave), 2) : cdiv(Tq, kWave);
-    dim3 grid(static_cast<unsigned>(pairs), static_cast<unsigned>(H), static_cast<unsigned>(B));
-#define SPARDA_ROUTE(KM_)                                                                          \
-    hipLaunchKernelGGL((route_rows_kernel<FDT, DF, KM_>), grid, dim3(kRouteThreads), 0, stream,    \
+    const int64_t sets = cdiv(Tq, kWave);
+    // Sets in pairs only where there are more than workgroups that run at once:
+    // below that a pair's second set waits for its first (12/4 heads, top-8 of
+    // 64-key blocks, us paired / single: T=512 10.0 / 6.8, T=4096 11.5 / 7.9; B=4,
+    // T=2048 10.3 / 7.9, T=4096 14.5 / 15.8; 32-key blocks T=8192 20.6 / 22.1).
+    const bool paired = causal && B * H * sets > (sets <= 64 ? 512 : 256);
+    dim3 grid(static_cast<unsigned>(paired ? cdiv(sets, 2) : sets), static_cast<unsigned>(H), static_cast<unsigned>(B));
+#define SPARDA_ROUTE(KM_, TB_)                                                                     \
+    hipLaunchKernelGGL((route_rows_kernel<FDT, DF, KM_, TB_>), grid, dim3(kRouteThreads), 0, stream, \
                        f, fsb, fst, fsh, protos, Tq, static_cast<int>(H), NB,                      \
                        static_cast<int>(bs), ke, causal, score_pos0, query_pos0, scale,            \
                        topk, scores, sel, n_sel, cap)
-    if (ke <= 8) { SPARDA_ROUTE(8); }
-    else if (ke <= 16) { SPARDA_ROUTE(16); }
-    else { SPARDA_ROUTE(32); }
+    // two tiles of 16 blocks at a time, one where there is no second: us of two /
+    // one, 4 heads, top-8: T=64 5.0 / 4.4, T=1000 5.4 / 4.9 (16 blocks), T=2048 5.9 / 6.3
+    if (NB <= 16) {
+        if (ke <= 8) { SPARDA_ROUTE(8, 1); }
+        else { SPARDA_ROUTE(16, 1); }
+    }
+    else if (ke <= 8) { SPARDA_ROUTE(8, 2); }
+    else if (ke <= 16) { SPARDA_ROUTE(16, 2); }
+    else { SPARDA_ROUTE(32, 2); }
 #undef SPARDA_ROUTE
     return check_hip(hipGetLastError(), "route_rows_kernel");
 }

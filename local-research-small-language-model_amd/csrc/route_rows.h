@@ -76,12 +76,13 @@ struct RouteShape {
 // l % 16, keeps that row's KMAX best route keys of its blocks, and the four
 // lanes of a row merge their lists at the end. On return best[rt] of a score
 // wavefront holds the list of row 16 (RT p + rt) + l % 16 over its block
-// group's blocks (merged further by the caller where BG > 1). With scores
+// group's blocks (merged further by the caller where BG > 1), in lanes 0..15, and
+// with ALL in the other lanes too. With scores
 // non-null every score of the row (-inf where masked) is written to
 // scores[row * NB]. Called by every wavefront of the workgroup (barriers
 // inside; `lds` holds Shape::kFloats floats and is free again after the
 // caller's next barrier).
-template <int FDT, int DF, int KMAX, int NW, int PG, int BG, int RT, int TB>
+template <int FDT, int DF, int KMAX, int NW, int PG, int BG, int RT, int TB, bool ALL>
 __device__ __forceinline__ void route_tiles(const void* __restrict__ f, int64_t fsb, int64_t fst, int64_t fsh,
                                             const float* __restrict__ protos, int b, int h, int H, int64_t row0,
                                             int nrows, int64_t Tq, int64_t NB, int bs, int causal,
@@ -134,13 +135,13 @@ __device__ __forceinline__ void route_tiles(const void* __restrict__ f, int64_t 
     const bool vec = (reinterpret_cast<uintptr_t>(f) & (FDT == SPARDA_F32 ? 15u : 7u)) == 0 && fsb % V == 0 &&
                      fst % V == 0 && fsh % V == 0;
     const int64_t fbase = b * fsb + h * fsh;
+    fetch(0);  // under the forecast's way through LDS
     for (int e = tid; e < Shape::kRows * kS; e += Shape::kThreads) {
         int64_t t = row0 + e / kS;
         t = t < t_last ? t : t_last;
         *reinterpret_cast<float4*>(lds + (e / kS) * kRow + 4 * (e % kS)) =
             load_forecast4<FDT>(f, fbase + t * fst + 4 * (e % kS), vec);
     }
-    fetch(0);
     __syncthreads();
     float fr[RT][kS];
     int limit[RT];
@@ -222,8 +223,8 @@ __device__ __forceinline__ void route_tiles(const void* __restrict__ f, int64_t 
         if (srow[rt] != nullptr && bg == 0)
             for (int64_t j = limit[rt] + 1 + grp; j < NB; j += 4) srow[rt][j] = -__builtin_inff();
         if (scorer && 16 * TB * bg <= jmax) {  // wave-uniform: the others' lists are empty
-            merge_rows<16>(best[rt]);
-            merge_rows<32>(best[rt]);
+            if (ALL || jmax >= 4) merge_rows<16>(best[rt]);  // fewer blocks sit in the first lanes alone
+            if (ALL || jmax >= 8) merge_rows<32>(best[rt]);
         }
     }
 }

@@ -1,5 +1,5 @@
 """The router's matrix-core scores against the oracle's fma chain, bit for bit:
-row sets and block chunks at their edges, every forecast
+row sets (alone and in pairs) and block chunks at their edges, every forecast
 width, and forecasts with denormal, cancelling, infinite and NaN elements and of
 mixed magnitude (where a chain differs from any other order of the sum)."""
 
@@ -18,6 +18,8 @@ DEV = "cuda"
 @pytest.mark.parametrize("Tq,NB,Df,k,causal,kind", [
     (1, 1, 64, 1, True, "normal"), (63, 2, 16, 2, True, "normal"), (65, 15, 32, 8, False, "normal"),
     (129, 17, 64, 8, True, "normal"), (200, 33, 128, 16, False, "normal"), (1000, 49, 64, 32, True, "normal"),
+    (70, 3, 64, 4, False, "normal"), (70, 4, 64, 4, True, "normal"), (70, 5, 64, 8, False, "normal"),
+    (70, 8, 64, 8, False, "normal"), (70, 9, 64, 8, False, "normal"), (70, 16, 128, 16, True, "normal"), (4161, 17, 16, 8, True, "normal"),
     (130, 70, 64, 8, False, "cancelling"), (130, 70, 128, 8, True, "mixed"), (130, 70, 16, 8, False, "mixed"),
     (130, 97, 64, 8, False, "tiny"), (130, 64, 64, 8, False, "infinite"), (130, 40, 64, 4, False, "equal")])
 def test_route_scores_and_lists(Tq, NB, Df, k, causal, kind):
