@@ -304,6 +304,12 @@ bool prefill_f32_supported(int dtype, int64_t T, int64_t Hq, int64_t Hkv, int64_
                            int64_t kv_st, int64_t kv_sh, int64_t out_sb, int64_t out_st, const void* q,
                            const void* k, const void* v, const void* out) {
     if (dtype != SPARDA_F32 || D != 64 || (bs != 64 && bs != 32) || Hq % Hkv != 0 || Hq / Hkv > 16) return false;
+    // short prompts in few workgroups go to the general kernel, which has one
+    // memory latency less before its keys and little else to do: us there / here
+    // for 6/2 heads, T=1 4.0 / 6.4, T=16 4.9 / 6.8, T=33 6.2 / 7.3, T=64 8.2 / 7.1;
+    // 32-key blocks T=16 5.0 / 5.6, T=33 7.2 / 5.7; 16/2 heads T=16 6.5 / 6.9, T=33
+    // 8.1 / 7.0; B=64, T=16 9.9 / 8.0.
+    if (T * (Hq / Hkv > 4 ? 4 : 1) <= (bs == 64 ? 40 : 16) && B * Hkv * T <= 512) return false;
     // a tile's list entries are counted in 32 bits, its blocks in the mask array
     if (sel != nullptr && (cdiv(T, bs) > kFMaxNB || cap >= (int64_t(1) << 27))) return false;
     if (B * Hkv * cdiv(T, 16 / (Hq / Hkv)) >= (int64_t(1) << 31)) return false;

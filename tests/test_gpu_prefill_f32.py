@@ -19,7 +19,10 @@ DEV = "cuda"
 @pytest.mark.parametrize("R,T,bs,k,causal,dense", [
     (1, 33, 64, 8, True, False), (3, 65, 32, 4, True, False), (3, 333, 64, 2, True, False),
     (4, 200, 32, 4, False, False), (5, 190, 64, 8, True, False), (16, 130, 32, 4, True, False),
-    (3, 127, 64, 8, True, True), (2, 97, 64, 8, False, True), (3, 1, 64, 8, True, True)])
+    (3, 127, 64, 8, True, True), (2, 97, 64, 8, False, True), (3, 1, 64, 8, True, True),
+    # either side of the lengths the general kernel keeps
+    (3, 40, 64, 8, True, False), (3, 41, 64, 8, True, True), (3, 41, 64, 8, True, False), (1, 16, 32, 4, True, False),
+    (1, 17, 32, 4, False, False), (8, 10, 64, 8, True, False), (8, 11, 64, 8, False, False)])
 def test_f32_prefill_against_the_oracle(R, T, bs, k, causal, dense):
     print(f"[case] f32 R={R} T={T} bs={bs} causal={causal} dense={dense}", flush=True)
     x = synth.prefill_inputs(2, T, 2 * R, 2, 64, dtype=torch.float32, seed=60 + T)
