@@ -24,7 +24,7 @@
 // hence four wavefronts per tile rather than more columns per wavefront. The
 // VALU kernel it stands in for served one token per workgroup through LDS: a
 // layer of T=1024, 12/4 heads, top-8 of 64-key blocks (compressor and router
-// included) 206 us then, 52 us now; T=2048 420 and 108.
+// included) 206 us then, 47 us now; T=2048 420 and 102 (the attention 38 and 92).
 //
 // A masked column's P is 0, but 0 x V is NaN where V is infinite or NaN: an
 // entry whose V holds such values is added token by token, with the rows that
