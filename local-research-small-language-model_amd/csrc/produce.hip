@@ -396,13 +396,14 @@ int launch_produce(const void* x, int64_t x_st, const void* w, int64_t M, int64_
         default: SPARDA_PRODUCE(FDT_, 2, 32); break;            \
     }
     // The widest tile that leaves the chip enough workgroups (N = 1536, C = 768):
-    // 256 rows past two workgroups per CU (62 us against 74 with 128 rows at
-    // M = 16384; 39.9 against 38.7 at 8192), 128 rows past one per CU (25.9 us
+    // 256 rows past two and a half workgroups per CU, two at a time (62 us against
+    // 68 with 128 rows at M = 16384, 3 per CU; 69 against 58 at 12000, 2.2 per CU,
+    // where a second round is nearly empty), 128 rows past one per CU (25.9 us
     // against 28.1 with 64 rows at 4096), 64 rows below (20.1 against 19.3 at 2048,
     // launch included). A width that is no multiple of 64 takes 32-wide steps.
     const int64_t cols = N / kPBN;
     const int tile = C % 64 != 0 ? (cdiv(M, 128) * cols > kPCus ? 3 : 4)
-                                 : (cdiv(M, 256) * cols > 2 * kPCus ? 0 : (cdiv(M, 128) * cols > kPCus ? 1 : 2));
+                                 : (2 * cdiv(M, 256) * cols > 5 * kPCus ? 0 : (cdiv(M, 128) * cols > kPCus ? 1 : 2));
     if (f_dtype == SPARDA_F32) { SPARDA_PRODUCE_T(SPARDA_F32) }
     else { SPARDA_PRODUCE_T(SPARDA_BF16) }
 #undef SPARDA_PRODUCE_T

@@ -14,7 +14,8 @@ DEV = "cuda"
 
 @pytest.mark.parametrize("B,T,C,nq,f_dtype", [(1, 63, 768, 768, torch.bfloat16), (1, 65, 96, 256, torch.float32),
                                               (3, 1820, 128, 768, torch.bfloat16), (1, 5500, 160, 1024, torch.float32),
-                                              (5, 2300, 64, 768, torch.bfloat16)])
+                                              (5, 2300, 64, 768, torch.bfloat16),
+                                              (5, 2783, 64, 768, torch.bfloat16)])  # 2.1, 2.6 workgroups a CU
 def test_produce_tile_edges(B, T, C, nq, f_dtype):
     print(f"[case] produce tiles B={B} T={T} C={C} nq={nq}", flush=True)
     g = torch.Generator().manual_seed(T)
